@@ -22,6 +22,7 @@ SOURCES = [
     ("refine.hip", ["-ffp-contract=off"]),
     ("sums.hip", ["-ffp-contract=off"]),
     ("nci.hip", ["-ffp-contract=fast"]),
+    ("fourier.hip", ["-ffp-contract=fast"]),
     ("ncigrid.hip", ["-ffp-contract=off"]),
     ("cube.hip", ["-ffp-contract=off"]),
     ("ncicut.hip", ["-ffp-contract=off"]),

@@ -399,6 +399,12 @@ __global__ void k_nci_fft_point(Geo G, const double *__restrict__ rho, const dou
 void nci_grid_launch(c2gpu_ctx *ctx, const Geo &G, const double x2c[9], const double c2x[9],
                      const double *d_rho, const NciOut &O);
 
+// line passes of the Fourier scheme (fourier.hip); the 3-D transforms here
+// serve grids with an edge too long for them
+bool fourier_lines_ok(const int n[3]);
+void fourier_lines_run(c2gpu_ctx *ctx, const double *f, const int n[3], const double bvec[9], int kind, double *out,
+                       const NciOut *O);
+
 static Geo make_geo(const int n[3], const double x2c[9]) {
   Geo G{};
   G.n1 = n[0];
@@ -741,8 +747,14 @@ void fft_deriv_run(c2gpu_ctx *ctx, const double *rho, const int n[3], const doub
   const size_t N = (size_t)n[0] * n[1] * n[2];
   hipStream_t st = ctx->stream;
   const double *d_rho = to_device_grid(ctx, rho, N, flags, "fft_rho");
-  double2 *spec = buf<double2>(ctx, "fft_spec", N), *w = buf<double2>(ctx, "fft_work", N);
   double *d_out = (flags & C2GPU_PTR_DEVICE) ? out : buf<double>(ctx, "fft_out", N);
+  if (fourier_lines_ok(n)) {
+    fourier_lines_run(ctx, d_rho, n, make_recip(n, x2c).bvec, kind, d_out, nullptr);
+    if (!(flags & C2GPU_PTR_DEVICE)) C2_HIP(hipMemcpyAsync(out, d_out, 8 * N, hipMemcpyDeviceToHost, st));
+    C2_HIP(hipStreamSynchronize(st));
+    return;
+  }
+  double2 *spec = buf<double2>(ctx, "fft_spec", N), *w = buf<double2>(ctx, "fft_work", N);
   FftPlan plan(ctx, n);
   const unsigned g = grid_for((int64_t)N, 256);
   const Recip R = make_recip(n, x2c);
@@ -1021,25 +1033,29 @@ void nci_run(c2gpu_ctx *ctx, const double *rho, const int n[3], const double x2c
   } else if (scheme == C2GPU_NCI_FFT) {
     if (precision != C2GPU_FP64) fail(C2GPU_ERR_UNSUPPORTED, "c2gpu_nci: FFT scheme runs in FP64");
     const double *d_rho = to_device_grid(ctx, rho, N, flags, "nci_rho");
-    double2 *spec = buf<double2>(ctx, "fft_spec", N), *w = buf<double2>(ctx, "fft_work", N);
-    double *gsq = buf<double>(ctx, "nci_gsq", N);
-    int8_t *npos = buf<int8_t>(ctx, "nci_npos", N);
-    FftPlan plan(ctx, n);
-    const Recip R = make_recip(n, x2c);
-    C2_LAUNCH(ctx, k_real_to_complex, dim3(g), dim3(256), 0, d_rho, spec, N);
-    HIPFFT_CHECK(hipfftExecZ2Z(plan.h, (hipfftDoubleComplex *)spec, (hipfftDoubleComplex *)spec, HIPFFT_FORWARD));
-    for (int c = 0; c < 3; c++) {  // |grad rho|^2 (ifformat_as_ft_grad)
-      C2_LAUNCH(ctx, k_spectral, dim3(g), dim3(256), 0, R, spec, w, N, c);
-      HIPFFT_CHECK(hipfftExecZ2Z(plan.h, (hipfftDoubleComplex *)w, (hipfftDoubleComplex *)w, HIPFFT_BACKWARD));
-      C2_LAUNCH(ctx, k_accum_sq, dim3(g), dim3(256), 0, w, gsq, N, c == 0);
-    }
-    for (int c = 0; c < 3; c++) {  // xx, yy, zz signs
-      C2_LAUNCH(ctx, k_spectral, dim3(g), dim3(256), 0, R, spec, w, N, 10 + c);
-      HIPFFT_CHECK(hipfftExecZ2Z(plan.h, (hipfftDoubleComplex *)w, (hipfftDoubleComplex *)w, HIPFFT_BACKWARD));
-      C2_LAUNCH(ctx, k_count_pos, dim3(g), dim3(256), 0, w, npos, N, c == 0);
-    }
     if (out_f32) fail(C2GPU_ERR_UNSUPPORTED, "c2gpu_nci_f32: FFT scheme writes FP64");
-    C2_LAUNCH(ctx, k_nci_fft_point, dim3(g), dim3(256), 0, G, d_rho, gsq, npos, O);
+    if (fourier_lines_ok(n)) {
+      fourier_lines_run(ctx, d_rho, n, make_recip(n, x2c).bvec, -1, nullptr, &O);
+    } else {
+      double2 *spec = buf<double2>(ctx, "fft_spec", N), *w = buf<double2>(ctx, "fft_work", N);
+      double *gsq = buf<double>(ctx, "nci_gsq", N);
+      int8_t *npos = buf<int8_t>(ctx, "nci_npos", N);
+      FftPlan plan(ctx, n);
+      const Recip R = make_recip(n, x2c);
+      C2_LAUNCH(ctx, k_real_to_complex, dim3(g), dim3(256), 0, d_rho, spec, N);
+      HIPFFT_CHECK(hipfftExecZ2Z(plan.h, (hipfftDoubleComplex *)spec, (hipfftDoubleComplex *)spec, HIPFFT_FORWARD));
+      for (int c = 0; c < 3; c++) {  // |grad rho|^2 (ifformat_as_ft_grad)
+        C2_LAUNCH(ctx, k_spectral, dim3(g), dim3(256), 0, R, spec, w, N, c);
+        HIPFFT_CHECK(hipfftExecZ2Z(plan.h, (hipfftDoubleComplex *)w, (hipfftDoubleComplex *)w, HIPFFT_BACKWARD));
+        C2_LAUNCH(ctx, k_accum_sq, dim3(g), dim3(256), 0, w, gsq, N, c == 0);
+      }
+      for (int c = 0; c < 3; c++) {  // xx, yy, zz signs
+        C2_LAUNCH(ctx, k_spectral, dim3(g), dim3(256), 0, R, spec, w, N, 10 + c);
+        HIPFFT_CHECK(hipfftExecZ2Z(plan.h, (hipfftDoubleComplex *)w, (hipfftDoubleComplex *)w, HIPFFT_BACKWARD));
+        C2_LAUNCH(ctx, k_count_pos, dim3(g), dim3(256), 0, w, npos, N, c == 0);
+      }
+      C2_LAUNCH(ctx, k_nci_fft_point, dim3(g), dim3(256), 0, G, d_rho, gsq, npos, O);
+    }
   } else if (scheme == C2GPU_NCI_GRID) {
     if (precision != C2GPU_FP64) fail(C2GPU_ERR_UNSUPPORTED, "c2gpu_nci: grid scheme runs in FP64");
     for (int c = 0; c < 3; c++)

@@ -1,0 +1,67 @@
+"""The Fourier derivative grids over the edges at which their line transforms
+change (radices, circulant edges, tile remainders, the longest line, the 3-D
+transform beyond it) and over cell shapes, against the oracle's numpy FFT.
+
+The fields are white noise, whose second derivatives are of the size of the
+largest multiplier, so the round-off of either side is a few tens of 2.2e-16
+of the largest value (the circulant sums grow as sqrt(n)): 1e-12 of it is
+asserted."""
+import numpy as np
+import pytest
+
+from critic2_amd import _lib
+from critic2_amd import bader as gb
+from critic2_amd import nci as gn
+from critic2_amd.synth import lattice_from_params
+from oracle import oracle
+
+pytestmark = pytest.mark.gpu
+
+ORTHO = np.diag([7.0, 8.0, 9.0])
+TRI = lattice_from_params(7.0, 8.0, 9.0, 80, 100, 110)
+MONO = lattice_from_params(7.0, 8.0, 9.0, 90, 105, 90)
+PERM = np.array([[0.0, 0.0, 9.0], [-7.0, 0.0, 0.0], [0.0, 8.0, 0.0]])  # axes along z, x (negative), y
+CELLS = {"ortho": ORTHO, "ortho_angles": lattice_from_params(7.0, 8.0, 9.0, 90, 90, 90), "triclinic": TRI,
+         "monoclinic": MONO, "permuted": PERM}
+GRIDS = [
+    (1, 2, 3), (2, 2, 2), (3, 1, 4), (5, 4, 7),   # the smallest edges
+    (16, 15, 17), (17, 33, 31), (18, 49, 10),      # remainders of the 16-column tiles; primes
+    (64, 9, 35), (11, 128, 22), (26, 13, 96),      # circulant edges, even and odd, on each axis
+    (512, 6, 5), (3, 640, 4), (6, 5, 1024), (101, 4, 1001),  # fewer line pairs a workgroup
+    (3375, 3, 2), (2, 3, 2048), (3391, 2, 3),      # near the longest line
+    (3500, 3, 2),                                  # the 3-D transform
+]
+
+
+@pytest.mark.parametrize("grid", GRIDS)
+@pytest.mark.parametrize("cell", ["ortho_angles", "triclinic"])
+def test_edges(ctx, cell, grid):
+    print(f"[case] fourier {cell} {grid}", flush=True)
+    f = np.random.default_rng(sum(grid)).normal(size=int(np.prod(grid)))
+    for kind, name in ((_lib.FT_GRAD, "grad"), (_lib.FT_YY, "yy"), (_lib.FT_LAP, "lap")):
+        g = gb.fft_deriv(ctx, f, grid, CELLS[cell], kind)
+        o = oracle.fft_deriv(f, grid, CELLS[cell], name)
+        assert np.abs(g - o).max() <= 1e-12 * max(np.abs(o).max(), 1e-3), name
+
+
+@pytest.mark.parametrize("cell", sorted(CELLS))
+@pytest.mark.parametrize("grid", [(12, 14, 18), (15, 20, 11), (21, 9, 25)])
+def test_cells(ctx, cell, grid):
+    """Every kind and nciplot's node values in both layouts."""
+    print(f"[case] fourier {cell} {grid}", flush=True)
+    f = 0.1 + np.random.default_rng(sum(grid)).uniform(size=int(np.prod(grid)))
+    x2c = CELLS[cell]
+    d = {}
+    for kind, name in ((_lib.FT_GRAD, "grad"), (_lib.FT_XX, "xx"), (_lib.FT_YY, "yy"), (_lib.FT_ZZ, "zz"),
+                       (_lib.FT_LAP, "lap")):
+        d[name] = oracle.fft_deriv(f, grid, x2c, name)
+        assert np.abs(gb.fft_deriv(ctx, f, grid, x2c, kind) - d[name]).max() <= 1e-12 * np.abs(d[name]).max(), name
+    crho, s = gn.nciplot_grid(ctx, f, grid, x2c, zfast=False)
+    ref = d["grad"] / (2 * (3 * np.pi ** 2) ** (1 / 3) * f ** (4 / 3))
+    np.testing.assert_allclose(s, ref, rtol=1e-10, atol=1e-12 * ref.max())
+    up = sum((d[q] > 0).astype(int) for q in ("xx", "yy", "zz"))
+    clear = np.min([np.abs(d[q]) / np.abs(d[q]).max() for q in ("xx", "yy", "zz")], axis=0) > 1e-11
+    assert np.array_equal(crho[clear], np.where(up >= 2, f, -f)[clear] * 100.0)
+    cz, sz = gn.nciplot_grid(ctx, f, grid, x2c)
+    for z, x in ((cz, crho), (sz, s)):
+        assert np.array_equal(z.reshape(grid), x.reshape(grid[::-1]).transpose(2, 1, 0))
