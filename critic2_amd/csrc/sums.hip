@@ -6,7 +6,7 @@
 // wavefront takes 64 consecutive points, forms runs of equal labels with a
 // segmented scan over the lanes (labels are spatially coherent, so runs are
 // long), and the run tails add into the workgroup's LDS bins one after the
-// other.  Block partials go to HBM and a second kernel adds them in block
+// other.  Block partials go to HBM and a second kernel adds them in a fixed
 // order, so the result is bitwise reproducible for a given grid size.
 #include <hip/hip_runtime.h>
 
@@ -115,13 +115,37 @@ __global__ void __launch_bounds__(64 * SUM_WAVES)
   for (uint64_t t = b0 + (uint64_t)wave * 64; t < b1; t += 64 * SUM_WAVES) tile_sums(lab, t, b1, nattr, nf, F, wb);
 }
 
-__global__ void k_basin_reduce(const double *__restrict__ partial, int nblocks, int nb,
-                               double *__restrict__ out) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= nb) return;
+// The total of bin q over the block partials, for a workgroup of RED_COLS
+// bins x RED_ROWS rows: row r adds blocks r, r + RED_ROWS, ... in order, and
+// the rows are added in order, so the result depends on nblocks alone.  One
+// thread per bin adding 2048 blocks one after the other was a chain of 2048
+// loads: 242 us for 16 bins x 1024 blocks, 485 us for 148 x 2048 (200x192x240,
+// 74 atoms); now below 7 and 10 us.  Every thread calls it; the total is
+// valid in row 0 of a bin below nb.
+static constexpr int RED_COLS = 16, RED_ROWS = 64;
+__device__ __forceinline__ double fold_blocks(const double *__restrict__ partial, int nblocks, int nb, int q) {
+  __shared__ double part[RED_ROWS][RED_COLS];
+  const int c = threadIdx.x % RED_COLS, r = threadIdx.x / RED_COLS;
   double s = 0.0;
-  for (int b = 0; b < nblocks; b++) s += partial[(size_t)b * nb + q];
-  out[q] = s;
+  if (q < nb) {
+#pragma unroll 8
+    for (int b = r; b < nblocks; b += RED_ROWS) s += partial[(size_t)b * nb + q];
+  }
+  part[r][c] = s;
+  __syncthreads();
+  double t = 0.0;
+  if (r == 0) {
+#pragma unroll 16
+    for (int k = 0; k < RED_ROWS; k++) t += part[k][c];
+  }
+  return t;
+}
+
+__global__ void __launch_bounds__(RED_COLS *RED_ROWS)
+    k_basin_reduce(const double *__restrict__ partial, int nblocks, int nb, double *__restrict__ out) {
+  const int q = blockIdx.x * RED_COLS + threadIdx.x % RED_COLS;
+  const double s = fold_blocks(partial, nblocks, nb, q);
+  if (threadIdx.x < RED_COLS && q < nb) out[q] = s;
 }
 
 __global__ void k_relabel(int32_t *__restrict__ lab, uint64_t npts, const int32_t *__restrict__ map,
@@ -168,7 +192,8 @@ void basin_sums_run(c2gpu_ctx *ctx, const int32_t *label, int64_t npts, int natt
     const size_t lds = sizeof(double) * (size_t)nb * SUM_WAVES;
     C2_LAUNCH(ctx, k_basin_partials, dim3(nblocks), dim3(64 * SUM_WAVES), lds, d_lab, (uint64_t)npts, nattr, nfields,
               F, chunk, partial);
-    C2_LAUNCH(ctx, k_basin_reduce, dim3(grid_for(nb, 256)), dim3(256), 0, partial, nblocks, nb, d_out);
+    C2_LAUNCH(ctx, k_basin_reduce, dim3((nb + RED_COLS - 1) / RED_COLS), dim3(RED_COLS * RED_ROWS), 0, partial,
+              nblocks, nb, d_out);
   } else {
     // fewer, longer chunks keep the rows (8 bytes x bins x 4 per block) to
     // at most about 1 GiB
@@ -184,7 +209,8 @@ void basin_sums_run(c2gpu_ctx *ctx, const int32_t *label, int64_t npts, int natt
     C2_HIP(hipMemsetAsync(rowsb, 0, sizeof(double) * (size_t)nblocks * SUM_WAVES * nb, st));
     C2_LAUNCH(ctx, k_basin_partials_rows, dim3(nblocks), dim3(64 * SUM_WAVES), 0, d_lab, (uint64_t)npts, nattr,
               nfields, F, chunk, rowsb);
-    C2_LAUNCH(ctx, k_basin_reduce, dim3(grid_for(nb, 256)), dim3(256), 0, rowsb, nblocks * SUM_WAVES, nb, d_out);
+    C2_LAUNCH(ctx, k_basin_reduce, dim3((nb + RED_COLS - 1) / RED_COLS), dim3(RED_COLS * RED_ROWS), 0, rowsb,
+              nblocks * SUM_WAVES, nb, d_out);
   }
   std::vector<double> h(nb);
   copy_to_host(ctx, h.data(), d_out, 8 * (size_t)nb);
@@ -223,16 +249,16 @@ void noalloc_init(int device) {
   scratch_dev[device] = static_cast<double *>(p);
 }
 
-// The block partials in bin order, added in block order (as k_basin_reduce),
-// written straight to the caller's outputs: counts (bins 0..nattr-1) as
-// int64, then each field's sums.
-__global__ void k_basin_reduce_out(const double *__restrict__ partial, int nblocks, int nattr, int nf,
-                                   double *__restrict__ sums_out, int64_t *__restrict__ counts_out) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+// The block partials added as k_basin_reduce adds them, written straight to
+// the caller's outputs: counts (bins 0..nattr-1) as int64, then each field's
+// sums.
+__global__ void __launch_bounds__(RED_COLS *RED_ROWS)
+    k_basin_reduce_out(const double *__restrict__ partial, int nblocks, int nattr, int nf,
+                       double *__restrict__ sums_out, int64_t *__restrict__ counts_out) {
+  const int q = blockIdx.x * RED_COLS + threadIdx.x % RED_COLS;
   const int nb = (nf + 1) * nattr;
-  if (q >= nb) return;
-  double s = 0.0;
-  for (int b = 0; b < nblocks; b++) s += partial[(size_t)b * nb + q];
+  const double s = fold_blocks(partial, nblocks, nb, q);
+  if (threadIdx.x >= RED_COLS || q >= nb) return;
   if (q < nattr) {
     if (counts_out) counts_out[q] = (int64_t)s;
   } else {
@@ -274,8 +300,8 @@ void basin_sums_noalloc_run(c2gpu_ctx *ctx, const int32_t *label, int64_t npts, 
   hipLaunchKernelGGL(k_basin_partials, dim3(nblocks), dim3(64 * SUM_WAVES), lds, ctx->stream, label,
                      (uint64_t)npts, nattr, nfields, F, chunk, partial);
   C2_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_basin_reduce_out, dim3((nb + 255) / 256), dim3(256), 0, ctx->stream, partial, nblocks,
-                     nattr, nfields, sums_out, counts_out);
+  hipLaunchKernelGGL(k_basin_reduce_out, dim3((nb + RED_COLS - 1) / RED_COLS), dim3(RED_COLS * RED_ROWS), 0, ctx->stream,
+                     partial, nblocks, nattr, nfields, sums_out, counts_out);
   C2_HIP(hipGetLastError());
 }
 
