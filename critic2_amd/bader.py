@@ -138,7 +138,15 @@ def basin_sums(ctx: Context, labels, nattr: int, fields=()):
 
 
 def fft_deriv(ctx: Context, rho, n, x2c, kind):
-    """grid3%fft (grid3mod@proc.f90:1757-1872) on a host grid."""
+    """grid3%fft (grid3mod@proc.f90:1757-1872) on a host grid (numpy array
+    back), or on a grid in HBM (DeviceArray back)."""
+    if hasattr(rho, "data_ptr") and getattr(rho, "is_cuda", True):
+        out = ctx.empty((int(np.prod(n)),), np.float64)
+        nn = np.asarray(n, dtype=np.int32)
+        x = _lib.mat_f(x2c)
+        ctx.check(ctx.lib.c2gpu_fft_deriv(ctx.h, _lib.ptr(rho), nn.ctypes.data, x.ctypes.data, kind,
+                                          _lib.PTR_DEVICE, _lib.ptr(out)), "c2gpu_fft_deriv")
+        return out
     rho = np.ascontiguousarray(rho, dtype=np.float64).reshape(-1)
     out = np.zeros_like(rho)
     nn = np.asarray(n, dtype=np.int32)
@@ -158,11 +166,7 @@ def intgrid_fields(ctx: Context, bas: BasinData, rho, x2c, lap=True):
     omega = abs(float(np.linalg.det(np.asarray(x2c))))
     fields = [rho]
     if lap:
-        host_rho = rho.numpy() if hasattr(rho, "data_ptr") else rho
-        lapg = fft_deriv(ctx, host_rho, n, x2c, _lib.FT_LAP)
-        if hasattr(rho, "data_ptr"):
-            lapg = ctx.to_device(lapg)
-        fields.append(lapg)
+        fields.append(fft_deriv(ctx, rho, n, x2c, _lib.FT_LAP))
     counts, sums = basin_sums(ctx, bas.idg, bas.nattr, fields)
     w = omega / npts
     out = {"volume": counts * w, "pop": sums[0] * w}
@@ -275,9 +279,18 @@ def reorder_map(xattr, x2c, cpcel, cptyp, nat_atoms, ratom, atexist=True):
 
 
 def bader(ctx: Context, rho, n, x2c, xat, nnm=False, ratom=None, noatoms=False, lap=True):
-    """BADER keyword: labels + attractors + integrated Volume/Pop/Lap."""
+    """BADER keyword: labels + attractors + integrated Volume/Pop/Lap.  A host
+    grid crosses to the GPU once for the whole keyword, its labels back once."""
+    host = not hasattr(rho, "data_ptr")
+    if host:
+        rho = np.ascontiguousarray(rho, dtype=np.float64).reshape(-1)
+        if rho.size != int(np.prod(n)):
+            raise ValueError(f"rho holds {rho.size} values, the grid {tuple(n)} has {int(np.prod(n))}")
+        rho = ctx.to_device(rho)
     bas = bader_integrate(ctx, rho, n, x2c, xat, nnm=nnm, ratom=ratom, noatoms=noatoms)
     props = intgrid_fields(ctx, bas, rho, x2c, lap=lap)
+    if host:
+        bas.idg = bas.idg.numpy()
     return bas, props
 
 

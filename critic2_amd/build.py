@@ -30,6 +30,7 @@ SOURCES = [
     ("mpole.hip", ["-ffp-contract=off"]),
     ("wscell.cpp", ["-ffp-contract=off"]),
     ("qcksort.cpp", ["-ffp-contract=off"]),
+    ("hostcopy.cpp", ["-ffp-contract=off"]),
     ("batch.cpp", ["-ffp-contract=off"]),
     ("capi.cpp", ["-ffp-contract=off"]),
 ]

@@ -270,7 +270,7 @@ void bader_run(c2gpu_ctx *ctx, const double *rho, const int n[3], const double c
   const double *d_rho = rho;
   if (!(flags & C2GPU_PTR_DEVICE)) {
     double *d = buf<double>(ctx, "bader_rho", N);
-    C2_HIP(hipMemcpyAsync(d, rho, sizeof(double) * N, hipMemcpyHostToDevice, st));
+    copy_in(ctx, d, rho, sizeof(double) * N);
     d_rho = d;
   }
   BParams P = make_params(d_rho, n, car2lat, lat_i_dist);
@@ -465,7 +465,7 @@ void bader_run(c2gpu_ctx *ctx, const double *rho, const int n[3], const double c
   if (flags & C2GPU_PTR_DEVICE)
     C2_HIP(hipMemcpyAsync(label_out, V, sizeof(int32_t) * N, hipMemcpyDeviceToDevice, st));
   else
-    C2_HIP(hipMemcpyAsync(label_out, V, sizeof(int32_t) * N, hipMemcpyDeviceToHost, st));
+    copy_out(ctx, label_out, V, sizeof(int32_t) * N);
   C2_HIP(hipStreamSynchronize(st));
   S.nattr = nbasin;
   if (nattr) *nattr = nbasin;
@@ -489,7 +489,7 @@ void step_pointers_run(c2gpu_ctx *ctx, const double *rho, const int n[3], const 
   const double *d_rho = rho;
   if (!dev) {
     double *d = buf<double>(ctx, "sp_rho", N);
-    C2_HIP(hipMemcpyAsync(d, rho, sizeof(double) * N, hipMemcpyHostToDevice, st));
+    copy_in(ctx, d, rho, sizeof(double) * N);
     d_rho = d;
   }
   int64_t *d_on = ongrid, *d_ne = near0;
@@ -502,9 +502,9 @@ void step_pointers_run(c2gpu_ctx *ctx, const double *rho, const int n[3], const 
   BParams P = make_params(d_rho, n, car2lat, lat_i_dist);
   C2_LAUNCH(ctx, k_step_pointers, dim3(grid_for(N, 256)), dim3(256), 0, P, N, d_on, d_ne, d_dr);
   if (!dev) {
-    if (ongrid) C2_HIP(hipMemcpyAsync(ongrid, d_on, 8 * (size_t)N, hipMemcpyDeviceToHost, st));
-    if (near0) C2_HIP(hipMemcpyAsync(near0, d_ne, 8 * (size_t)N, hipMemcpyDeviceToHost, st));
-    if (dr1) C2_HIP(hipMemcpyAsync(dr1, d_dr, 24 * (size_t)N, hipMemcpyDeviceToHost, st));
+    if (ongrid) copy_out(ctx, ongrid, d_on, 8 * (size_t)N);
+    if (near0) copy_out(ctx, near0, d_ne, 8 * (size_t)N);
+    if (dr1) copy_out(ctx, dr1, d_dr, 24 * (size_t)N);
   }
   C2_HIP(hipStreamSynchronize(st));
 }

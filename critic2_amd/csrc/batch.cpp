@@ -48,7 +48,7 @@ static void bader_cell(c2gpu_ctx *w, const c2gpu_cell &C, int attr_mode, double 
   const double *d_rho = C.rho;
   if (!dev) {
     double *d = buf<double>(w, "batch_rho", N);
-    C2_HIP(hipMemcpyAsync(d, C.rho, 8 * N, hipMemcpyHostToDevice, w->stream));
+    copy_in(w, d, C.rho, 8 * N);
     d_rho = d;
   }
   int32_t *d_lab = dev ? C.label_out : buf<int32_t>(w, "batch_lab", N);
@@ -72,7 +72,7 @@ static void bader_cell(c2gpu_ctx *w, const c2gpu_cell &C, int attr_mode, double 
     if (C.sums_out) std::memcpy(C.sums_out, sums.data(), sizeof(double) * nattr);
     if (C.counts_out) std::memcpy(C.counts_out, counts.data(), sizeof(int64_t) * nattr);
   }
-  if (!dev) C2_HIP(hipMemcpyAsync(C.label_out, d_lab, 4 * N, hipMemcpyDeviceToHost, w->stream));
+  if (!dev) copy_out(w, C.label_out, d_lab, 4 * N);
   C2_HIP(hipStreamSynchronize(w->stream));
 }
 

@@ -339,12 +339,13 @@ int c2gpu_dev_free(c2gpu_ctx *ctx, void *ptr) {
 
 int c2gpu_memcpy(c2gpu_ctx *ctx, void *dst, const void *src, uint64_t bytes, int kind) {
   return guarded(ctx, [&] {
-    hipMemcpyKind k = kind == 1 ? hipMemcpyHostToDevice
-                      : kind == 2 ? hipMemcpyDeviceToHost
-                      : kind == 3 ? hipMemcpyDeviceToDevice
-                                  : hipMemcpyDefault;
     if (kind < 1 || kind > 3) fail(C2GPU_ERR_ARG, "c2gpu_memcpy: bad kind");
-    C2_HIP(hipMemcpyAsync(dst, src, bytes, k, ctx->stream));
+    if (kind == 1)
+      copy_in(ctx, dst, src, bytes);
+    else if (kind == 2)
+      copy_out(ctx, dst, src, bytes);
+    else
+      C2_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, ctx->stream));
     C2_HIP(hipStreamSynchronize(ctx->stream));
   });
 }

@@ -47,6 +47,12 @@ struct c2gpu_ctx {
   // device address itself
   void *pin = nullptr;
   size_t pin_bytes = 0;
+  // pinned slots of the staged large host transfers (hostcopy.cpp)
+  static constexpr int STAGE_SLOTS = 6;
+  struct Stage {
+    void *ptr = nullptr;
+    hipEvent_t ev = nullptr;
+  } stage[STAGE_SLOTS];
   // the surface weights of the last c2gpu_yt call (context buffers
   // yt_ias, yt_woff, yt_wc, yt_wb, yt_ww), for c2gpu_yt_multipoles, as
   // critic2 keeps them in its YT checkpoint for later yt_weights calls
@@ -188,7 +194,17 @@ inline void add_kernel_bytes(c2gpu_ctx *ctx, const char *name, double bytes) {
     }                                                                          \
   } while (0)
 
+// Transfers of caller arrays and files, ordered on the context's stream
+// (hostcopy.cpp).  copy_in / file_in return when the source may change,
+// copy_out / file_out when the destination holds the data.
+void copy_in(c2gpu_ctx *ctx, void *dst, const void *src, size_t bytes);
+void copy_out(c2gpu_ctx *ctx, void *dst, const void *src, size_t bytes);
+void file_in(c2gpu_ctx *ctx, void *dst, int fd, uint64_t from, uint64_t bytes);
+void file_out(c2gpu_ctx *ctx, int fd, uint64_t to, const void *src, uint64_t bytes);
+void release_stage(c2gpu_ctx *ctx);
+
 inline void release_all(c2gpu_ctx *ctx) {
+  release_stage(ctx);
   for (auto &kv : ctx->bufs)
     if (kv.second.ptr) (void)hipFree(kv.second.ptr);
   ctx->bufs.clear();

@@ -20,10 +20,11 @@
 // fewer values, non-numeric tokens and list-directed forms other than plain
 // blank-separated constants (r*c repeats, commas, slashes) are errors.
 #include <hip/hip_runtime.h>
+#include <sys/stat.h>
 
+#include <algorithm>
 #include <cstdio>
 #include <cstring>
-#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -579,30 +580,6 @@ double *out_grid(c2gpu_ctx *ctx, int flags, double *f, uint64_t npts) {
   return buf<double>(ctx, "cube_out", npts);
 }
 
-// Pinned staging for host->device streaming of files.
-struct Pinned {
-  void *p[2] = {nullptr, nullptr};
-  hipEvent_t ev[2] = {nullptr, nullptr};
-  size_t bytes = 0;
-  explicit Pinned(size_t b) : bytes(b) {
-    for (int i = 0; i < 2; i++) {
-      C2_HIP(hipHostMalloc(&p[i], b, hipHostMallocDefault));
-      C2_HIP(hipEventCreateWithFlags(&ev[i], hipEventDisableTiming));
-    }
-  }
-  ~Pinned() {
-    for (int i = 0; i < 2; i++) {
-      if (ev[i]) {
-        (void)hipEventSynchronize(ev[i]);
-        (void)hipEventDestroy(ev[i]);
-      }
-      if (p[i]) (void)hipHostFree(p[i]);
-    }
-  }
-};
-
-constexpr size_t CHUNK = 64ull << 20;
-
 struct File {
   FILE *fp = nullptr;
   explicit File(const char *path) {
@@ -621,33 +598,11 @@ struct File {
   }
 };
 
-// Reads bytes [from, from + len) of fp into device memory dst, through
-// double-buffered pinned chunks.
-void stream_to_device(c2gpu_ctx *ctx, FILE *fp, uint64_t from, uint64_t len, uint8_t *dst) {
-  if (len == 0) return;
-  Pinned pin(len < CHUNK ? len : CHUNK);
-  fseeko(fp, (off_t)from, SEEK_SET);
-  uint64_t done = 0;
-  int which = 0;
-  bool used[2] = {false, false};
-  while (done < len) {
-    const size_t want = (size_t)((len - done) < pin.bytes ? (len - done) : pin.bytes);
-    if (used[which]) C2_HIP(hipEventSynchronize(pin.ev[which]));
-    if (fread(pin.p[which], 1, want, fp) != want) fail(C2GPU_ERR_FORMAT, "short read");
-    C2_HIP(hipMemcpyAsync(dst + done, pin.p[which], want, hipMemcpyHostToDevice, ctx->stream));
-    C2_HIP(hipEventRecord(pin.ev[which], ctx->stream));
-    used[which] = true;
-    done += want;
-    which ^= 1;
-  }
-  C2_HIP(hipStreamSynchronize(ctx->stream));
-}
-
-// Reads the text header of a file: the first MiB, growing until the header
-// is complete.
+// Reads the text header of a file: the first 64 KiB, growing until the
+// header is complete.
 void file_text_header(FILE *fp, uint64_t fsize, c2gpu_cube_header &h) {
   std::vector<char> b;
-  uint64_t want = 1ull << 20;
+  uint64_t want = 1ull << 16;
   for (;;) {
     const uint64_t n = want < fsize ? want : fsize;
     b.resize(n);
@@ -758,9 +713,9 @@ void cube_parse_run(c2gpu_ctx *ctx, const char *text, uint64_t len, int flags, c
     parse_values(ctx, base, lo, lo + (len - off), h->n, out);
   } else {
     uint8_t *d = buf<uint8_t>(ctx, "cube_text", len - off + 16);
-    C2_HIP(hipMemcpyAsync(d, text + off, len - off, hipMemcpyHostToDevice, ctx->stream));
+    copy_in(ctx, d, text + off, len - off);
     parse_values(ctx, d, 0, len - off, h->n, out);
-    C2_HIP(hipMemcpyAsync(f, out, npts * 8, hipMemcpyDeviceToHost, ctx->stream));
+    copy_out(ctx, f, out, npts * 8);
   }
   C2_HIP(hipStreamSynchronize(ctx->stream));
 }
@@ -775,10 +730,10 @@ void cube_read_run(c2gpu_ctx *ctx, const char *path, int flags, c2gpu_cube_heade
   double *out = out_grid(ctx, flags, f, npts);
   const uint64_t len = fsize - h->data_offset;
   uint8_t *d = buf<uint8_t>(ctx, "cube_text", len + 16);
-  stream_to_device(ctx, file.fp, h->data_offset, len, d);
+  if (len) file_in(ctx, d, fileno(file.fp), h->data_offset, len);
   parse_values(ctx, d, 0, len, h->n, out);
   if (!(flags & C2GPU_PTR_DEVICE))
-    C2_HIP(hipMemcpyAsync(f, out, npts * 8, hipMemcpyDeviceToHost, ctx->stream));
+    copy_out(ctx, f, out, npts * 8);
   C2_HIP(hipStreamSynchronize(ctx->stream));
 }
 
@@ -793,29 +748,16 @@ void bincube_read_run(c2gpu_ctx *ctx, const char *path, int flags, c2gpu_cube_he
   const bool dev = flags & C2GPU_PTR_DEVICE;
   if (dev) require_device_ptr(f, "f");
   uint64_t got = 0;
-  std::unique_ptr<Pinned> pin;
-  int which = 0;
-  bool used[2] = {false, false};
   r.read([&](uint64_t len) {
     // the grid record: the first npts doubles go to f, the rest is skipped
     uint64_t take = got < need ? (need - got < len ? need - got : len) : 0;
     if (!dev) {
       if (take && fread(reinterpret_cast<char *>(f) + got, 1, take, file.fp) != take)
         fail(C2GPU_ERR_FORMAT, "binary cube: end of file");
-    } else {
-      if (!pin && take) pin.reset(new Pinned(need < CHUNK ? need : CHUNK));
-      uint64_t done = 0;
-      while (done < take) {
-        const size_t want = (size_t)((take - done) < pin->bytes ? (take - done) : pin->bytes);
-        if (used[which]) C2_HIP(hipEventSynchronize(pin->ev[which]));
-        if (fread(pin->p[which], 1, want, file.fp) != want) fail(C2GPU_ERR_FORMAT, "binary cube: end of file");
-        C2_HIP(hipMemcpyAsync(reinterpret_cast<char *>(f) + got + done, pin->p[which], want,
-                              hipMemcpyHostToDevice, ctx->stream));
-        C2_HIP(hipEventRecord(pin->ev[which], ctx->stream));
-        used[which] = true;
-        done += want;
-        which ^= 1;
-      }
+    } else if (take) {
+      const off_t at = ftello(file.fp);
+      file_in(ctx, reinterpret_cast<char *>(f) + got, fileno(file.fp), (uint64_t)at, take);
+      fseeko(file.fp, at + (off_t)take, SEEK_SET);
     }
     got += take;
     if (len > take) fseeko(file.fp, (off_t)(len - take), SEEK_CUR);
@@ -843,10 +785,10 @@ void cube_format_run(c2gpu_ctx *ctx, const double *f, const int n[3], int style,
     format_body(ctx, f, n, style, zfast, text);
   } else {
     double *df = buf<double>(ctx, "cube_fin", npts);
-    C2_HIP(hipMemcpyAsync(df, f, npts * 8, hipMemcpyHostToDevice, ctx->stream));
+    copy_in(ctx, df, f, npts * 8);
     char *dt = buf<char>(ctx, "cube_text_out", nb);
     format_body(ctx, df, n, style, zfast, dt);
-    C2_HIP(hipMemcpyAsync(text, dt, nb, hipMemcpyDeviceToHost, ctx->stream));
+    copy_out(ctx, text, dt, nb);
   }
   C2_HIP(hipStreamSynchronize(ctx->stream));
 }
@@ -870,7 +812,7 @@ void cube_write_run(c2gpu_ctx *ctx, const char *path, const c2gpu_cube_header *h
       format_body(ctx, f, h->n, style, 0, dt);
     } else {
       double *df = buf<double>(ctx, "cube_fin", npts);
-      C2_HIP(hipMemcpyAsync(df, f, npts * 8, hipMemcpyHostToDevice, ctx->stream));
+      copy_in(ctx, df, f, npts * 8);
       format_body(ctx, df, h->n, style, 0, dt);
     }
   }
@@ -883,31 +825,17 @@ void cube_write_run(c2gpu_ctx *ctx, const char *path, const c2gpu_cube_header *h
     }
   } closer{fp};
   if (fwrite(head.data(), 1, head.size(), fp) != head.size()) fail(C2GPU_ERR_FORMAT, "cube: write failed");
-  if (nb) {
-    Pinned pin(nb < CHUNK ? nb : CHUNK);
-    uint64_t done = 0;
-    int which = 0;
-    // copy chunk c+1 while chunk c is written
-    size_t pending = 0;
-    int pend_buf = -1;
-    while (done < nb || pend_buf >= 0) {
-      size_t want = 0;
-      if (done < nb) {
-        want = (size_t)((nb - done) < pin.bytes ? (nb - done) : pin.bytes);
-        C2_HIP(hipMemcpyAsync(pin.p[which], dt + done, want, hipMemcpyDeviceToHost, ctx->stream));
-        C2_HIP(hipEventRecord(pin.ev[which], ctx->stream));
-      }
-      if (pend_buf >= 0) {
-        if (fwrite(pin.p[pend_buf], 1, pending, fp) != pending) fail(C2GPU_ERR_FORMAT, "cube: write failed");
-        pend_buf = -1;
-      }
-      if (want) {
-        C2_HIP(hipEventSynchronize(pin.ev[which]));
-        pending = want;
-        pend_buf = which;
-        done += want;
-        which ^= 1;
-      }
+  struct stat fs;
+  if (nb && fflush(fp) != 0) fail(C2GPU_ERR_FORMAT, "cube: write failed");
+  if (nb && fstat(fileno(fp), &fs) == 0 && S_ISREG(fs.st_mode)) {
+    file_out(ctx, fileno(fp), head.size(), dt, nb);
+  } else if (nb) {  // a pipe: in order
+    std::vector<char> part(std::min<uint64_t>(nb, 16ull << 20));
+    for (uint64_t done = 0; done < nb;) {
+      const size_t want = (size_t)std::min<uint64_t>(part.size(), nb - done);
+      copy_out(ctx, part.data(), dt + done, want);
+      if (fwrite(part.data(), 1, want, fp) != want) fail(C2GPU_ERR_FORMAT, "cube: write failed");
+      done += want;
     }
   }
   if (fclose(fp) != 0) {

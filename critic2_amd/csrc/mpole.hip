@@ -253,8 +253,8 @@ void mpole_impl(c2gpu_ctx *ctx, const char *who, bool yt, const int32_t *label, 
   } else {
     int32_t *dl = buf<int32_t>(ctx, "mp_lab", npts);
     double *df = buf<double>(ctx, "mp_f", npts);
-    C2_HIP(hipMemcpyAsync(dl, label, 4 * npts, hipMemcpyHostToDevice, st));
-    C2_HIP(hipMemcpyAsync(df, f, 8 * npts, hipMemcpyHostToDevice, st));
+    copy_in(ctx, dl, label, 4 * npts);
+    copy_in(ctx, df, f, 8 * npts);
     d_lab = dl;
     d_f = df;
   }

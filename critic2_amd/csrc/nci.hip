@@ -550,7 +550,7 @@ void synth_slater_run(c2gpu_ctx *ctx, const double x2c[9], const int n[3], int n
   C2_LAUNCH(ctx, k_slater, dim3(G.nb1 * G.nb2 * G.nb3), dim3(256), 0, G, d_img, d_zp,
                      rimg, BL.off, BL.lst, d_out);
   if (!(flags & C2GPU_PTR_DEVICE))
-    C2_HIP(hipMemcpyAsync(rho_out, d_out, 8 * N, hipMemcpyDeviceToHost, ctx->stream));
+    copy_out(ctx, rho_out, d_out, 8 * N);
   C2_HIP(hipStreamSynchronize(ctx->stream));
 }
 
@@ -735,7 +735,7 @@ static const double *to_device_grid(c2gpu_ctx *ctx, const double *rho, size_t N,
                                     const char *name) {
   if (flags & C2GPU_PTR_DEVICE) return rho;
   double *d = buf<double>(ctx, name, N);
-  C2_HIP(hipMemcpyAsync(d, rho, 8 * N, hipMemcpyHostToDevice, ctx->stream));
+  copy_in(ctx, d, rho, 8 * N);
   return d;
 }
 
@@ -750,7 +750,7 @@ void fft_deriv_run(c2gpu_ctx *ctx, const double *rho, const int n[3], const doub
   double *d_out = (flags & C2GPU_PTR_DEVICE) ? out : buf<double>(ctx, "fft_out", N);
   if (fourier_lines_ok(n)) {
     fourier_lines_run(ctx, d_rho, n, make_recip(n, x2c).bvec, kind, d_out, nullptr);
-    if (!(flags & C2GPU_PTR_DEVICE)) C2_HIP(hipMemcpyAsync(out, d_out, 8 * N, hipMemcpyDeviceToHost, st));
+    if (!(flags & C2GPU_PTR_DEVICE)) copy_out(ctx, out, d_out, 8 * N);
     C2_HIP(hipStreamSynchronize(st));
     return;
   }
@@ -773,7 +773,7 @@ void fft_deriv_run(c2gpu_ctx *ctx, const double *rho, const int n[3], const doub
     HIPFFT_CHECK(hipfftExecZ2Z(plan.h, (hipfftDoubleComplex *)w, (hipfftDoubleComplex *)w, HIPFFT_BACKWARD));
     C2_LAUNCH(ctx, k_real_part, dim3(g), dim3(256), 0, w, d_out, N);
   }
-  if (!(flags & C2GPU_PTR_DEVICE)) C2_HIP(hipMemcpyAsync(out, d_out, 8 * N, hipMemcpyDeviceToHost, st));
+  if (!(flags & C2GPU_PTR_DEVICE)) copy_out(ctx, out, d_out, 8 * N);
   C2_HIP(hipStreamSynchronize(st));
 }
 
@@ -999,8 +999,8 @@ void batch_nci_run(c2gpu_ctx *ctx, int ncell, const c2gpu_cell *cells, int nspec
     for (size_t q = 0; q < hc.size(); q++) {
       const c2gpu_cell &C = cells[sel[q]];
       const size_t npt = (size_t)C.n[0] * C.n[1] * C.n[2];
-      C2_HIP(hipMemcpyAsync(C.crho_out, stage + stage_at[q], 4 * npt, hipMemcpyDeviceToHost, st));
-      C2_HIP(hipMemcpyAsync(C.cgrad_out, stage + nstage + stage_at[q], 4 * npt, hipMemcpyDeviceToHost, st));
+      copy_out(ctx, C.crho_out, stage + stage_at[q], 4 * npt);
+      copy_out(ctx, C.cgrad_out, stage + nstage + stage_at[q], 4 * npt);
     }
   }
   C2_HIP(hipStreamSynchronize(st));
@@ -1066,8 +1066,8 @@ void nci_run(c2gpu_ctx *ctx, const double *rho, const int n[3], const double x2c
     fail(C2GPU_ERR_UNSUPPORTED, "c2gpu_nci: unknown scheme");
   }
   if (!dev) {
-    C2_HIP(hipMemcpyAsync(crho_out, O.crho, osz * N, hipMemcpyDeviceToHost, st));
-    C2_HIP(hipMemcpyAsync(cgrad_out, O.cgrad, osz * N, hipMemcpyDeviceToHost, st));
+    copy_out(ctx, crho_out, O.crho, osz * N);
+    copy_out(ctx, cgrad_out, O.cgrad, osz * N);
   }
   C2_HIP(hipStreamSynchronize(st));
 }
@@ -1150,9 +1150,9 @@ void nci_promol_nodes_run(c2gpu_ctx *ctx, const c2gpu_nci_nodes *nd, const doubl
   else
     C2_LAUNCH(ctx, k_promol_d, dim3(nbk), dim3(256), 0, G, P.D, P.img, BL.off, BL.lst, O);
   if (!dev) {
-    C2_HIP(hipMemcpyAsync(crho_out, O.crho, osz * N, hipMemcpyDeviceToHost, st));
-    C2_HIP(hipMemcpyAsync(cgrad_out, O.cgrad, osz * N, hipMemcpyDeviceToHost, st));
-    if (rhoat_out) C2_HIP(hipMemcpyAsync(rhoat_out, O.rhoat, osz * N, hipMemcpyDeviceToHost, st));
+    copy_out(ctx, crho_out, O.crho, osz * N);
+    copy_out(ctx, cgrad_out, O.cgrad, osz * N);
+    if (rhoat_out) copy_out(ctx, rhoat_out, O.rhoat, osz * N);
   }
   C2_HIP(hipStreamSynchronize(st));
 }
@@ -1259,7 +1259,7 @@ void nci_fragments_run(c2gpu_ctx *ctx, const c2gpu_nci_nodes *nd, int nspecies, 
   else
     C2_LAUNCH(ctx, k_frag<double>, dim3(g), dim3(256), 0, G, P.D, P.F, (const double4 *)d_at, (const int *)d_fs,
               nfrag, npts, (double *)out);
-  if (!dev) C2_HIP(hipMemcpyAsync(rhofrag_out, out, osz * npts * nfrag, hipMemcpyDeviceToHost, st));
+  if (!dev) copy_out(ctx, rhofrag_out, out, osz * npts * nfrag);
   C2_HIP(hipStreamSynchronize(st));
 }
 

@@ -196,15 +196,15 @@ void cut_entry(c2gpu_ctx *ctx, const void *crho_, void *cgrad_, const void *rhoa
     T *dc = buf<T>(ctx, "ncicut_crho", npts);
     T *dg = buf<T>(ctx, "ncicut_cgrad", npts);
     T *da = nullptr;
-    C2_HIP(hipMemcpyAsync(dc, crho, npts * sizeof(T), hipMemcpyHostToDevice, ctx->stream));
-    C2_HIP(hipMemcpyAsync(dg, cgrad, npts * sizeof(T), hipMemcpyHostToDevice, ctx->stream));
+    copy_in(ctx, dc, crho, npts * sizeof(T));
+    copy_in(ctx, dg, cgrad, npts * sizeof(T));
     if (use_at) {
       da = buf<T>(ctx, "ncicut_rhoat", npts);
-      C2_HIP(hipMemcpyAsync(da, rhoat, npts * sizeof(T), hipMemcpyHostToDevice, ctx->stream));
+      copy_in(ctx, da, rhoat, npts * sizeof(T));
     }
     if (nfrag > 0) {
       T *df = buf<T>(ctx, "ncicut_rhofrag", npts * (uint64_t)nfrag);
-      C2_HIP(hipMemcpyAsync(df, F.rf, npts * (uint64_t)nfrag * sizeof(T), hipMemcpyHostToDevice, ctx->stream));
+      copy_in(ctx, df, F.rf, npts * (uint64_t)nfrag * sizeof(T));
       F.rf = df;
     }
     char *dd = nullptr;
@@ -212,8 +212,8 @@ void cut_entry(c2gpu_ctx *ctx, const void *crho_, void *cgrad_, const void *rhoa
       const uint64_t c = cap < npts * (uint64_t)ROW ? cap : npts * (uint64_t)ROW;
       dd = buf<char>(ctx, "ncicut_dat", c > 0 ? c : 1);
       cut_run<T>(ctx, npts, dc, dg, da, F, o, dd, c, len, sums);
-      if (*len) C2_HIP(hipMemcpyAsync(dat, dd, *len, hipMemcpyDeviceToHost, ctx->stream));
-      C2_HIP(hipMemcpyAsync(cgrad, dg, npts * sizeof(T), hipMemcpyDeviceToHost, ctx->stream));
+      if (*len) copy_out(ctx, dat, dd, *len);
+      copy_out(ctx, cgrad, dg, npts * sizeof(T));
     } else {
       cut_run<T>(ctx, npts, dc, dg, da, F, o, nullptr, 0, len, sums);
     }

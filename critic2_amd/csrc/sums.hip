@@ -169,11 +169,11 @@ void basin_sums_run(c2gpu_ctx *ctx, const int32_t *label, int64_t npts, int natt
   FieldPtrs F{};
   if (!dev) {
     int32_t *d = buf<int32_t>(ctx, "sum_lab", npts);
-    C2_HIP(hipMemcpyAsync(d, label, 4 * (size_t)npts, hipMemcpyHostToDevice, st));
+    copy_in(ctx, d, label, 4 * (size_t)npts);
     d_lab = d;
     for (int q = 0; q < nfields; q++) {
       double *df = buf<double>(ctx, "sum_f" + std::to_string(q), npts);
-      C2_HIP(hipMemcpyAsync(df, fields[q], 8 * (size_t)npts, hipMemcpyHostToDevice, st));
+      copy_in(ctx, df, fields[q], 8 * (size_t)npts);
       F.p[q] = df;
     }
   } else {
@@ -314,12 +314,12 @@ void relabel_run(c2gpu_ctx *ctx, int64_t npts, const int32_t *map, int nmap, int
   int32_t *d_lab = label;
   if (!(flags & C2GPU_PTR_DEVICE)) {
     d_lab = buf<int32_t>(ctx, "relabel_lab", npts);
-    C2_HIP(hipMemcpyAsync(d_lab, label, 4 * (size_t)npts, hipMemcpyHostToDevice, st));
+    copy_in(ctx, d_lab, label, 4 * (size_t)npts);
   }
   C2_LAUNCH(ctx, k_relabel, dim3(grid_for(npts, 256)), dim3(256), 0, d_lab,
                      (uint64_t)npts, d_map, nmap);
   if (!(flags & C2GPU_PTR_DEVICE))
-    C2_HIP(hipMemcpyAsync(label, d_lab, 4 * (size_t)npts, hipMemcpyDeviceToHost, st));
+    copy_out(ctx, label, d_lab, 4 * (size_t)npts);
   C2_HIP(hipStreamSynchronize(st));
 }
 

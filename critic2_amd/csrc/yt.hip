@@ -686,11 +686,11 @@ void yt_run(c2gpu_ctx *ctx, const double *rho, const int n[3], const double x2c[
     if (label_out) require_device_ptr(label_out, "label_out");
   } else {
     double *d = buf<double>(ctx, "yt_rho", N);
-    C2_HIP(hipMemcpyAsync(d, rho, 8 * (size_t)N, hipMemcpyHostToDevice, st));
+    copy_in(ctx, d, rho, 8 * (size_t)N);
     g = d;
     for (int q = 0; q < nfields; q++) {
       double *df = buf<double>(ctx, "yt_f" + std::to_string(q), N);
-      C2_HIP(hipMemcpyAsync(df, fields[q], 8 * (size_t)N, hipMemcpyHostToDevice, st));
+      copy_in(ctx, df, fields[q], 8 * (size_t)N);
       F.p[q] = df;
     }
   }
@@ -721,7 +721,7 @@ void yt_run(c2gpu_ctx *ctx, const double *rho, const int n[3], const double x2c[
     h_rk.assign(N, 0);
     for (uint32_t q = 0; q < N; q++) h_rk[io[q]] = q;
     uint32_t *d_rk = buf<uint32_t>(ctx, "yt_rank", N);
-    C2_HIP(hipMemcpyAsync(d_rk, h_rk.data(), 4 * (size_t)N, hipMemcpyHostToDevice, st));
+    copy_in(ctx, d_rk, h_rk.data(), 4 * (size_t)N);
     C2_HIP(hipStreamSynchronize(st));
     G.rk = d_rk;
     S.ranked = 1;
@@ -875,7 +875,7 @@ void yt_run(c2gpu_ctx *ctx, const double *rho, const int n[3], const double x2c[
   }
   std::vector<double> h(nb);
   copy_to_host(ctx, h.data(), acc, 8 * nb);
-  if (label_out && !dev) C2_HIP(hipMemcpyAsync(label_out, lab, 4 * (size_t)N, hipMemcpyDeviceToHost, st));
+  if (label_out && !dev) copy_out(ctx, label_out, lab, 4 * (size_t)N);
   C2_HIP(hipStreamSynchronize(st));
   for (int a = 0; a < nattr; a++) vol_out[a] = (double)counts[a] + h[a];
   for (int q = 0; q < nfields; q++)

@@ -10,12 +10,33 @@ crystallographic coordinates c2x (x0 - molx0) (:540-541).
 from __future__ import annotations
 
 import ctypes as C
+import mmap
 import os
 
 import numpy as np
 
 from . import _lib
 from ._lib import Context, CubeHeader
+
+
+_PyBytes_New = C.pythonapi.PyBytes_FromStringAndSize
+_PyBytes_New.restype, _PyBytes_New.argtypes = C.py_object, [C.c_void_p, C.c_ssize_t]
+_PyBytes_Address = C.pythonapi.PyBytes_AsString
+_PyBytes_Address.restype, _PyBytes_Address.argtypes = C.c_void_p, [C.py_object]
+_HUGE = 2 << 20
+
+
+def _text_buffer(size: int):
+    """A bytes object of `size` bytes, its contents not yet written, and its
+    address.  Large ones ask for 2 MiB pages: touching 386 MB for the first
+    time 4 KiB at a time cost 11 of the copy's 19 ms."""
+    out = _PyBytes_New(None, size)
+    p = _PyBytes_Address(out)
+    lo, hi = -(-p // _HUGE) * _HUGE, (p + size) // _HUGE * _HUGE
+    madvise = getattr(C.CDLL(None), "madvise", None)
+    if hi - lo >= 8 * _HUGE and madvise is not None:
+        madvise(C.c_void_p(lo), C.c_size_t(hi - lo), getattr(mmap, "MADV_HUGEPAGE", 14))  # a hint: may fail
+    return out, p
 
 
 def _header_dict(h: CubeHeader, x2c=None, molx0=None) -> dict:
@@ -96,17 +117,19 @@ def format_body(ctx: Context, f, n, style: int = _lib.CUBE_E22_14, zfast: bool =
     ln = C.c_uint64()
     ctx.check(ctx.lib.c2gpu_cube_format(ctx.h, None, nn.ctypes.data, style, int(zfast), 0, None, 0, C.byref(ln)),
               "c2gpu_cube_format")
-    out = np.empty(ln.value, dtype=np.uint8)
+    # the text goes straight into the bytes object returned
+    out, p = _text_buffer(ln.value)
     if hasattr(f, "data_ptr"):
         d = ctx.empty((ln.value,), np.uint8)
         ctx.check(ctx.lib.c2gpu_cube_format(ctx.h, f.data_ptr(), nn.ctypes.data, style, int(zfast),
                                             _lib.PTR_DEVICE, d.data_ptr(), ln.value, C.byref(ln)),
                   "c2gpu_cube_format")
-        return d.numpy().tobytes()
+        ctx.check(ctx.lib.c2gpu_memcpy(ctx.h, p, d.data_ptr(), ln.value, 2), "c2gpu_memcpy")
+        return out
     f = np.ascontiguousarray(f, dtype=np.float64).reshape(-1)
     ctx.check(ctx.lib.c2gpu_cube_format(ctx.h, f.ctypes.data, nn.ctypes.data, style, int(zfast), 0,
-                                        out.ctypes.data, ln.value, C.byref(ln)), "c2gpu_cube_format")
-    return out.tobytes()
+                                        p, ln.value, C.byref(ln)), "c2gpu_cube_format")
+    return out
 
 
 def write_cube(ctx: Context, path: str, n, x0, step, zat=(), xat=(), f=None, style: int = _lib.CUBE_E22_14):
