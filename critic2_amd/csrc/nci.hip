@@ -4,11 +4,11 @@
 // (crystalmod@env.f90:622-753, grid1mod@proc.f90:86-137), and the synthetic
 // Slater-sum grid used as test and benchmark input.
 //
-// Atom-sum kernels work on bricks of 8x8x4 grid nodes (one 256-thread
-// workgroup per brick).  A brick's neighbour list holds the periodic atom
-// images whose cutoff sphere can reach the brick; lists are built in two
-// deterministic passes (count, scan, fill in image order), so every point
-// sums its atoms in a fixed order.
+// Atom-sum kernels work on bricks of 256 grid nodes (one workgroup each).  A
+// brick's neighbour list holds the periodic atom images whose cutoff sphere
+// can reach the brick, in image order, so every point sums its atoms in a
+// fixed order.  The promolecular kernels make it in LDS as they go; the
+// synthetic grid's lists are built in two passes (count, scan, fill).
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 #include <hipfft/hipfft.h>
@@ -32,9 +32,8 @@ struct Images {
 };
 
 __device__ __forceinline__ bool image_hits_brick(const Geo &G, const Images &I, int b, int m) {
-  const int b1 = b % G.nb1, b2 = (b / G.nb1) % G.nb2, b3 = b / (G.nb1 * G.nb2);
   double c[3];
-  geo_cart(G, b1 * BX + 0.5 * (BX - 1), b2 * BY + 0.5 * (BY - 1), b3 * BZ + 0.5 * (BZ - 1), c);
+  brick_middle(G, b, c);
   const double4 p = I.pos[m];
   const double dx = p.x - c[0], dy = p.y - c[1], dz = p.z - c[2];
   const double rr = I.rcut[(int)p.w] + I.brad;
@@ -61,6 +60,50 @@ __global__ void __launch_bounds__(64) k_brick_list(Geo G, Images I, uint32_t *__
   if (!out && lane == 0) cnt[b] = total;
 }
 
+// The images that can reach a brick, in image order, STAGE_CAP at most at a
+// time in LDS: all of the workgroup's 256 threads test an image each, and the
+// hits keep their order (a prefix over the wavefronts' ballots).  Testing every
+// image against every brick here is hidden in the 2.0 ms of the 512^3 FP32
+// kernel (2.0 before, too); lists in memory took two launches of 0.42 ms, a
+// scan and a read-back.
+constexpr int STAGE_CAP = 512;
+struct ImageStage {
+  double4 img[STAGE_CAP];
+  uint32_t cnt[2][4];
+};
+// Stages from image m on until the stage could overflow or the images end;
+// moves m past the images tested and returns the number staged.  Called by
+// every thread, the stage no longer being read; ready to be read on return.
+__device__ __forceinline__ int stage_images(const Images &I, const double c[3], int &m, ImageStage &S) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  int n = 0;
+  for (int flip = 0; m < I.nimg && n + 256 <= STAGE_CAP; m += 256, flip ^= 1) {
+    const int q = m + (int)threadIdx.x;
+    bool hit = false;
+    double4 p;
+    if (q < I.nimg) {
+      p = I.pos[q];
+      const double dx = p.x - c[0], dy = p.y - c[1], dz = p.z - c[2];
+      const double rr = I.rcut[(int)p.w] + I.brad;
+      hit = dx * dx + dy * dy + dz * dz <= rr * rr;
+    }
+    const uint64_t mask = __ballot(hit);
+    if (lane == 0) S.cnt[flip][w] = (uint32_t)__popcll(mask);
+    __syncthreads();
+    int before = 0, total = 0;
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int v = (int)S.cnt[flip][u];
+      before += u < w ? v : 0;
+      total += v;
+    }
+    if (hit) S.img[n + before + __popcll(mask & ((1ull << lane) - 1ull))] = p;
+    n += total;
+  }
+  __syncthreads();
+  return n;
+}
+
 // ---------------------------------------------------------------- synthetic grid
 
 __global__ void __launch_bounds__(256) k_slater(Geo G, const double4 *__restrict__ img,
@@ -71,7 +114,7 @@ __global__ void __launch_bounds__(256) k_slater(Geo G, const double4 *__restrict
   const int b = blockIdx.x;
   const int b1 = b % G.nb1, b2 = (b / G.nb1) % G.nb2, b3 = b / (G.nb1 * G.nb2);
   const int t = threadIdx.x;
-  const int i = b1 * BX + (t % BX), j = b2 * BY + ((t / BX) % BY), k = b3 * BZ + t / (BX * BY);
+  const int i = b1 * 8 + (t % 8), j = b2 * 8 + ((t / 8) % 8), k = b3 * 4 + t / 64;  // 8x8x4, x fastest
   if (i >= G.n1 || j >= G.n2 || k >= G.n3) return;
   double xc[3];
   node_cart(G, i, j, k, xc);
@@ -98,9 +141,22 @@ struct RadTabD {  // FP64 tables, exact grid1%interp
 
 struct PromolD {
   const double *r, *f, *fp, *fpp;  // concatenated tables
+  // 1/(r_i - r_j), j < i, of the four nodes from r on: (1,0) (2,0) (2,1)
+  // (3,0) (3,1) (3,2), six per node (k_table_inv)
+  const double *inv;
   const int *toff, *tng;           // per species offset / ngrid
   const double *ta, *tb, *trmax, *tcut;
 };
+
+// The reciprocal node differences of interp_d, once per call instead of six
+// divisions per atom and node: the same quotients.  Entries whose four nodes
+// run past their table are never read.
+__global__ void k_table_inv(int n, const double *__restrict__ r, double *__restrict__ inv) {
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= n) return;
+  for (int i = 1, e = 0; i < 4; i++)
+    for (int j = 0; j < i; j++, e++) inv[6 * (size_t)q + e] = q + 3 < n ? 1.0 / (r[q + i] - r[q + j]) : 0.0;
+}
 
 // grid1%interp (grid1mod@proc.f90:86-137), FP64, same operation order
 __device__ inline void interp_d(const PromolD &T, int s, double r0, double &f, double &fp,
@@ -122,21 +178,17 @@ __device__ inline void interp_d(const PromolD &T, int s, double r0, double &f, d
   }
   int base = ir < 2 ? 2 : ir;
   base = base > ng - 2 ? ng - 2 : base;
-  double rr[4], dr1[4], x[4][4];
+  double dr1[4], x[4][4];
+  const double *iv = T.inv + 6 * (size_t)(o + base - 2);
 #pragma unroll
   for (int i = 0; i < 4; i++) {
-    rr[i] = R[base - 2 + i];
-    dr1[i] = r - rr[i];
-#pragma unroll
-    for (int j = 0; j < 4; j++) x[i][j] = 0.0;
-  }
-#pragma unroll
-  for (int i = 0; i < 4; i++)
+    dr1[i] = r - R[base - 2 + i];
 #pragma unroll
     for (int j = 0; j < i; j++) {
-      x[i][j] = 1.0 / (rr[i] - rr[j]);
+      x[i][j] = iv[i * (i - 1) / 2 + j];
       x[j][i] = -x[i][j];
     }
+  }
 #pragma unroll
   for (int i = 0; i < 4; i++) {
     double prod = 1.0;
@@ -162,145 +214,149 @@ struct PromolF {
   const float *tlog_a;      // log(a)
   const float *tr0;         // r(1)
   const float *trmax;
+  const float *cut2;        // squared cutoff radius
   const float *tnode;       // node r(base-1) per [toff+base]
 };
 
-// FP64 promolecular NCI (nci@proc.f90:565-604 with crystalmod@env.f90:622-753)
-__global__ void __launch_bounds__(256) k_promol_d(Geo G, PromolD T, const double4 *__restrict__ img,
-                                                  const uint64_t *__restrict__ off,
-                                                  const uint32_t *__restrict__ lst, NciOut O) {
-  const int b = blockIdx.x;
-  const int b1 = b % G.nb1, b2 = (b / G.nb1) % G.nb2, b3 = b / (G.nb1 * G.nb2);
-  const int t = threadIdx.x;
-  const int i = b1 * BX + (t % BX), j = b2 * BY + ((t / BX) % BY), k = b3 * BZ + t / (BX * BY);
-  if (i >= G.n1 || j >= G.n2 || k >= G.n3) return;
-  double xc[3];
-  node_cart(G, i, j, k, xc);
-  double f = 0.0, g0 = 0.0, g1 = 0.0, g2 = 0.0;
-  double h00 = 0.0, h11 = 0.0, h22 = 0.0, h01 = 0.0, h02 = 0.0, h12 = 0.0;
+// Sums over the atoms at a node: density, gradient, Hessian.
+template <class T>
+struct AtomSums {
+  T f = 0, g0 = 0, g1 = 0, g2 = 0, h00 = 0, h11 = 0, h22 = 0, h01 = 0, h02 = 0, h12 = 0;
   bool isnuc = false;
-  for (uint64_t q = off[b]; q < off[b + 1]; q++) {
-    const double4 p = img[lst[q]];
-    const int s = (int)p.w;
-    const double x0 = xc[0] - p.x, x1 = xc[1] - p.y, x2 = xc[2] - p.z;
-    double r = sqrt(x0 * x0 + x1 * x1 + x2 * x2);
-    if (r <= 1e-5) isnuc = true;  // identify_atom(distmax=1d-5), fieldmod@proc.f90:1148
-    if (r > T.tcut[s]) continue;
-    const double r1 = T.r[T.toff[s]];
-    r = r > r1 ? r : r1;
-    r = r > 1e-14 ? r : 1e-14;
-    double rho, rhop, rhopp;
-    interp_d(T, s, r, rho, rhop, rhopp);
-    rho = rho > 0.0 ? rho : 0.0;
-    f = f + rho;
-    const double rinv1 = 1.0 / r;
-    const double rinv1rp = rinv1 * rhop;
-    g0 = g0 + x0 * rinv1rp;
-    g1 = g1 + x1 * rinv1rp;
-    g2 = g2 + x2 * rinv1rp;
-    const double rfac = (rhopp - rinv1rp) * rinv1 * rinv1;
-    h00 = h00 + rinv1rp + rfac * x0 * x0;
-    h11 = h11 + rinv1rp + rfac * x1 * x1;
-    h22 = h22 + rinv1rp + rfac * x2 * x2;
-    h01 = h01 + rfac * x1 * x0;
-    h02 = h02 + rfac * x2 * x0;
-    h12 = h12 + rfac * x2 * x1;
-  }
-  if (isnuc) g0 = g1 = g2 = 0.0;
-  const double gmod = sqrt(g0 * g0 + g1 * g1 + g2 * g2);
-  const double cst = 2.0 * pow(3.0 * PI_D * PI_D, 1.0 / 3.0);
-  const double den = f > 1e-80 ? f : 1e-80;
-  const double s = gmod / (cst * pow(den, 4.0 / 3.0));
-  const double l2 = eig_mid_t<double>(h00, h11, h22, h01, h02, h12);
-  const double a = fabs(f) * 100.0;
-  const double crho = (l2 < 0.0 || (l2 == 0.0 && signbit(l2))) ? -a : a;
-  const size_t o = out_index(G, O.zfast, i, j, k);
-  store_out<double>(O, o, crho, s);
-  if (O.rhoat) ((double *)O.rhoat)[o] = f;
+};
+
+// The atom at p (w: species) added at node xc in FP64
+// (crystalmod@env.f90:622-753).
+__device__ __forceinline__ void add_atom(AtomSums<double> &A, const PromolD &T, const double4 &p,
+                                         const double xc[3]) {
+  const int s = __builtin_amdgcn_readfirstlane((int)p.w);  // one image for the whole wavefront
+  const double x0 = xc[0] - p.x, x1 = xc[1] - p.y, x2 = xc[2] - p.z;
+  double r = sqrt(x0 * x0 + x1 * x1 + x2 * x2);
+  if (r <= 1e-5) A.isnuc = true;  // identify_atom(distmax=1d-5), fieldmod@proc.f90:1148
+  if (r > T.tcut[s]) return;
+  const double r1 = T.r[T.toff[s]];
+  r = r > r1 ? r : r1;
+  r = r > 1e-14 ? r : 1e-14;
+  double rho, rhop, rhopp;
+  interp_d(T, s, r, rho, rhop, rhopp);
+  rho = rho > 0.0 ? rho : 0.0;
+  A.f = A.f + rho;
+  const double rinv1 = 1.0 / r;
+  const double rinv1rp = rinv1 * rhop;
+  A.g0 = A.g0 + x0 * rinv1rp;
+  A.g1 = A.g1 + x1 * rinv1rp;
+  A.g2 = A.g2 + x2 * rinv1rp;
+  const double rfac = (rhopp - rinv1rp) * rinv1 * rinv1;
+  A.h00 = A.h00 + rinv1rp + rfac * x0 * x0;
+  A.h11 = A.h11 + rinv1rp + rfac * x1 * x1;
+  A.h22 = A.h22 + rinv1rp + rfac * x2 * x2;
+  A.h01 = A.h01 + rfac * x1 * x0;
+  A.h02 = A.h02 + rfac * x2 * x0;
+  A.h12 = A.h12 + rfac * x2 * x1;
 }
 
-// FP32 promolecular NCI at node (i,j,k) from the image list lst[qb..qe)
-// (the atom sum of crystalmod@env.f90:622-753 and nci@proc.f90:565-599),
-// with per-interval cubic tables.  The node-atom difference is taken in
-// FP64 and then rounded: node and image coordinates reach tens of bohr,
-// where an FP32 coordinate is off by up to 4e-6 bohr, a relative density
-// error of about zeta * 4e-6 for an exponential tail; the rounded
-// difference is off by 6e-8 of itself.
-__device__ __forceinline__ void promol_f_node(const Geo &G, const PromolF &T, const double4 *__restrict__ img,
-                                              const float *__restrict__ cut2, const uint32_t *__restrict__ lst,
-                                              uint64_t qb, uint64_t qe, int i, int j, int k, const NciOut &O) {
-  double xcd[3];
-  node_cart(G, i, j, k, xcd);
-  float f = 0.f, g0 = 0.f, g1 = 0.f, g2 = 0.f;
-  float h00 = 0.f, h11 = 0.f, h22 = 0.f, h01 = 0.f, h02 = 0.f, h12 = 0.f;
-  bool isnuc = false;
-  for (uint64_t q = qb; q < qe; q++) {
-    const double4 p = img[lst[q]];
-    const int s = (int)p.w;
-    const float x0 = (float)(xcd[0] - p.x), x1 = (float)(xcd[1] - p.y), x2 = (float)(xcd[2] - p.z);
-    const float rsq = x0 * x0 + x1 * x1 + x2 * x2;
-    if (rsq <= 1e-10f) isnuc = true;
-    if (rsq > cut2[s]) continue;
-    float r = sqrtf(rsq);
-    if (r >= T.trmax[s]) continue;
-    const float r1 = T.tr0[s];
-    int ir;
-    if (r <= r1) {
-      ir = 1;
-      r = r1;
-    } else {
-      ir = 1 + (int)floorf((__logf(r) - T.tlog_a[s]) * T.ta_inv_b[s]);
-    }
-    const int ng = T.tng[s];
-    int base = ir < 2 ? 2 : ir;
-    base = base > ng - 2 ? ng - 2 : base;
-    const int ci = T.toff[s] + base;
-    const float u = r - T.tnode[ci];
-    const float4 cf = T.coef[4 * (size_t)ci + 0];  // f: c0..c3
-    const float4 cp = T.coef[4 * (size_t)ci + 1];  // fp
-    const float4 cq = T.coef[4 * (size_t)ci + 2];  // fpp
-    float rho = ((cf.w * u + cf.z) * u + cf.y) * u + cf.x;
-    const float rhop = ((cp.w * u + cp.z) * u + cp.y) * u + cp.x;
-    const float rhopp = ((cq.w * u + cq.z) * u + cq.y) * u + cq.x;
-    rho = rho > 0.f ? rho : 0.f;
-    f += rho;
-    const float rinv1 = 1.0f / r;
-    const float rinv1rp = rinv1 * rhop;
-    g0 += x0 * rinv1rp;
-    g1 += x1 * rinv1rp;
-    g2 += x2 * rinv1rp;
-    const float rfac = (rhopp - rinv1rp) * rinv1 * rinv1;
-    h00 += rinv1rp + rfac * x0 * x0;
-    h11 += rinv1rp + rfac * x1 * x1;
-    h22 += rinv1rp + rfac * x2 * x2;
-    h01 += rfac * x1 * x0;
-    h02 += rfac * x2 * x0;
-    h12 += rfac * x2 * x1;
+// nci@proc.f90:565-604 from the sums
+__device__ __forceinline__ void store_node(const AtomSums<double> &A, const NciOut &O, size_t o) {
+  const double g0 = A.isnuc ? 0.0 : A.g0, g1 = A.isnuc ? 0.0 : A.g1, g2 = A.isnuc ? 0.0 : A.g2;
+  const double gmod = sqrt(g0 * g0 + g1 * g1 + g2 * g2);
+  const double cst = 2.0 * pow(3.0 * PI_D * PI_D, 1.0 / 3.0);
+  const double den = A.f > 1e-80 ? A.f : 1e-80;
+  const double s = gmod / (cst * pow(den, 4.0 / 3.0));
+  const double a = fabs(A.f) * 100.0;
+  const double crho = eig_mid_negative<double>(A.h00, A.h11, A.h22, A.h01, A.h02, A.h12) ? -a : a;
+  store_out<double>(O, o, crho, s);
+  if (O.rhoat) ((double *)O.rhoat)[o] = A.f;
+}
+
+// The same in FP32 with per-interval cubic tables.  The node-atom difference
+// is taken in FP64 and then rounded: node and image coordinates reach tens of
+// bohr, where an FP32 coordinate is off by up to 4e-6 bohr, a relative density
+// error of about zeta * 4e-6 for an exponential tail; the rounded difference
+// is off by 6e-8 of itself.
+__device__ __forceinline__ void add_atom(AtomSums<float> &A, const PromolF &T, const double4 &p,
+                                         const double xc[3]) {
+  const int s = __builtin_amdgcn_readfirstlane((int)p.w);
+  const float x0 = (float)(xc[0] - p.x), x1 = (float)(xc[1] - p.y), x2 = (float)(xc[2] - p.z);
+  const float rsq = x0 * x0 + x1 * x1 + x2 * x2;
+  if (rsq <= 1e-10f) A.isnuc = true;
+  if (rsq > T.cut2[s]) return;
+  float r = sqrtf(rsq);
+  if (r >= T.trmax[s]) return;
+  const float r1 = T.tr0[s];
+  int ir;
+  if (r <= r1) {
+    ir = 1;
+    r = r1;
+  } else {
+    ir = 1 + (int)floorf((__logf(r) - T.tlog_a[s]) * T.ta_inv_b[s]);
   }
-  if (isnuc) g0 = g1 = g2 = 0.f;
+  const int ng = T.tng[s];
+  int base = ir < 2 ? 2 : ir;
+  base = base > ng - 2 ? ng - 2 : base;
+  const int ci = T.toff[s] + base;
+  const float u = r - T.tnode[ci];
+  const float4 cf = T.coef[4 * (size_t)ci + 0];  // f: c0..c3
+  const float4 cp = T.coef[4 * (size_t)ci + 1];  // fp
+  const float4 cq = T.coef[4 * (size_t)ci + 2];  // fpp
+  float rho = ((cf.w * u + cf.z) * u + cf.y) * u + cf.x;
+  const float rhop = ((cp.w * u + cp.z) * u + cp.y) * u + cp.x;
+  const float rhopp = ((cq.w * u + cq.z) * u + cq.y) * u + cq.x;
+  rho = rho > 0.f ? rho : 0.f;
+  A.f += rho;
+  const float rinv1 = 1.0f / r;
+  const float rinv1rp = rinv1 * rhop;
+  A.g0 += x0 * rinv1rp;
+  A.g1 += x1 * rinv1rp;
+  A.g2 += x2 * rinv1rp;
+  const float rfac = (rhopp - rinv1rp) * rinv1 * rinv1;
+  A.h00 += rinv1rp + rfac * x0 * x0;
+  A.h11 += rinv1rp + rfac * x1 * x1;
+  A.h22 += rinv1rp + rfac * x2 * x2;
+  A.h01 += rfac * x1 * x0;
+  A.h02 += rfac * x2 * x0;
+  A.h12 += rfac * x2 * x1;
+}
+
+__device__ __forceinline__ void store_node(const AtomSums<float> &A, const NciOut &O, size_t o) {
+  const float g0 = A.isnuc ? 0.f : A.g0, g1 = A.isnuc ? 0.f : A.g1, g2 = A.isnuc ? 0.f : A.g2;
   const float gmod = sqrtf(g0 * g0 + g1 * g1 + g2 * g2);
   // 2 (3 pi^2)^(1/3); max(rho, 1e-30f): 1d-80 is not representable in FP32
   const float cst = 6.18733545256027186f;
-  const float den = f > 1e-30f ? f : 1e-30f;
+  const float den = A.f > 1e-30f ? A.f : 1e-30f;
   const float s = gmod / (cst * den * cbrtf(den));
-  const float l2 = eig_mid_t<float>(h00, h11, h22, h01, h02, h12);
-  const float a = fabsf(f) * 100.f;
-  const float crho = (l2 < 0.f || (l2 == 0.f && signbit(l2))) ? -a : a;
-  const size_t o = out_index(G, O.zfast, i, j, k);
+  const float a = fabsf(A.f) * 100.f;
+  const float crho = eig_mid_negative<float>(A.h00, A.h11, A.h22, A.h01, A.h02, A.h12) ? -a : a;
   store_out<float>(O, o, crho, s);
-  if (O.rhoat) ((float *)O.rhoat)[o] = f;
+  if (O.rhoat) ((float *)O.rhoat)[o] = A.f;
 }
 
-__global__ void __launch_bounds__(256) k_promol_f(Geo G, PromolF T, const double4 *__restrict__ img,
-                                                  const float *__restrict__ cut2,
-                                                  const uint64_t *__restrict__ off,
-                                                  const uint32_t *__restrict__ lst, NciOut O) {
-  const int b = blockIdx.x;
-  const int b1 = b % G.nb1, b2 = (b / G.nb1) % G.nb2, b3 = b / (G.nb1 * G.nb2);
-  const int t = threadIdx.x;
-  const int i = b1 * BX + (t % BX), j = b2 * BY + ((t / BX) % BY), k = b3 * BZ + t / (BX * BY);
-  if (i >= G.n1 || j >= G.n2 || k >= G.n3) return;
-  promol_f_node(G, T, img, cut2, lst, off[b], off[b + 1], i, j, k, O);
+// The promolecular block on brick b, by the whole workgroup.
+template <class T, class Tab>
+__device__ __forceinline__ void promol_brick(const Geo &G, const Tab &tab, const Images &I, int b, const NciOut &O,
+                                             ImageStage &S) {
+  int i, j, k;
+  const bool in = brick_node(G, b, threadIdx.x, i, j, k);
+  double xc[3], c[3];
+  node_cart(G, i, j, k, xc);
+  brick_middle(G, b, c);
+  AtomSums<T> A;
+  for (int m = 0; m < I.nimg;) {
+    const int n = stage_images(I, c, m, S);
+    if (in)
+      for (int q = 0; q < n; q++) add_atom(A, tab, S.img[q], xc);
+    __syncthreads();  // the stage is filled again
+  }
+  if (in) store_node(A, O, out_index(G, O.zfast, i, j, k));
+}
+
+__global__ void __launch_bounds__(256) k_promol_d(Geo G, PromolD T, Images I, NciOut O) {
+  __shared__ ImageStage S;
+  promol_brick<double>(G, T, I, blockIdx.x, O, S);
+}
+
+__global__ void __launch_bounds__(256) k_promol_f(Geo G, PromolF T, Images I, NciOut O) {
+  __shared__ ImageStage S;
+  promol_brick<float>(G, T, I, blockIdx.x, O, S);
 }
 
 // ---------------------------------------------------------------- FFT scheme
@@ -405,21 +461,30 @@ bool fourier_lines_ok(const int n[3]);
 void fourier_lines_run(c2gpu_ctx *ctx, const double *f, const int n[3], const double bvec[9], int kind, double *out,
                        const NciOut *O);
 
-static Geo make_geo(const int n[3], const double x2c[9]) {
+// Bricks of 8x8x4 nodes, x fastest, or, where the outputs are z fastest, of
+// 4x8x8, z fastest: a wavefront then stores runs of 8 nodes, where lanes along
+// x put each of its nodes on a line of its own.  Longer runs (4x4x16, 4x2x32)
+// reach more atoms and lose more than the stores gain (512^3 FP32: 2.00 ms,
+// 2.20 and 2.29).
+static Geo make_geo(const int n[3], const double x2c[9], int zfast = 0) {
   Geo G{};
   G.n1 = n[0];
   G.n2 = n[1];
   G.n3 = n[2];
-  G.nb1 = (n[0] + BX - 1) / BX;
-  G.nb2 = (n[1] + BY - 1) / BY;
-  G.nb3 = (n[2] + BZ - 1) / BZ;
+  G.zf = zfast ? 1 : 0;
+  G.lx = zfast ? 2 : 3;
+  G.ly = 3;
+  G.lz = zfast ? 3 : 2;
+  G.nb1 = (n[0] + (1 << G.lx) - 1) >> G.lx;
+  G.nb2 = (n[1] + (1 << G.ly) - 1) >> G.ly;
+  G.nb3 = (n[2] + (1 << G.lz) - 1) >> G.lz;
   for (int q = 0; q < 9; q++) G.x2c[q] = x2c[q];
   return G;
 }
 
 // The nodes x0 + i xmat(:,1) + j xmat(:,2) + k xmat(:,3) of an nciplot cube.
 static Geo make_geo_box(const c2gpu_nci_nodes &nd, const double x2c[9]) {
-  Geo G = make_geo(nd.nstep, x2c);
+  Geo G = make_geo(nd.nstep, x2c, 1);
   G.box = 1;
   for (int r = 0; r < 3; r++) G.x0[r] = nd.x0[r];
   for (int q = 0; q < 9; q++) G.xm[q] = nd.xmat[q];
@@ -428,10 +493,11 @@ static Geo make_geo_box(const c2gpu_nci_nodes &nd, const double x2c[9]) {
 
 static double brick_radius(const Geo &G) {
   double h[3][3];
-  const double e[3] = {0.5 * (BX - 1) / G.n1, 0.5 * (BY - 1) / G.n2, 0.5 * (BZ - 1) / G.n3};
+  const double half[3] = {0.5 * ((1 << G.lx) - 1), 0.5 * ((1 << G.ly) - 1), 0.5 * ((1 << G.lz) - 1)};
+  const int n[3] = {G.n1, G.n2, G.n3};
   for (int a = 0; a < 3; a++)
-    for (int r = 0; r < 3; r++) h[a][r] = G.box ? G.xm[r + 3 * a] * (0.5 * ((a == 0 ? BX : a == 1 ? BY : BZ) - 1))
-                                                : G.x2c[r + 3 * a] * e[a];
+    for (int r = 0; r < 3; r++)
+      h[a][r] = G.box ? G.xm[r + 3 * a] * half[a] : G.x2c[r + 3 * a] * (half[a] / n[a]);
   double best = 0;
   for (int s = 0; s < 8; s++) {
     double v[3];
@@ -561,7 +627,6 @@ struct PromolDev {
   PromolF F;
   double4 *img;
   double *rcut;
-  float *cut2f;
   int nimg;
 };
 
@@ -664,7 +729,10 @@ static double upload_tables(c2gpu_ctx *ctx, int ns, const c2gpu_radial_table *ta
   P.F.trmax = (const float *)up("pm_trmaxf", trmaxf.data(), 4 * ns);
   P.F.tnode = (const float *)up("pm_node", node.data(), 4 * node.size());
   P.rcut = (double *)up("pm_rcut", tcut.data(), 8 * ns);
-  P.cut2f = (float *)up("pm_cut2", cut2.data(), 4 * ns);
+  P.F.cut2 = (const float *)up("pm_cut2", cut2.data(), 4 * ns);
+  double *inv = buf<double>(ctx, "pm_inv", 6 * (size_t)tot);
+  C2_LAUNCH(ctx, k_table_inv, dim3(grid_for(tot, 256)), dim3(256), 0, tot, P.D.r, inv);
+  P.D.inv = inv;
   C2_HIP(hipStreamSynchronize(ctx->stream));  // the host vectors end here
   return rcmax;
 }
@@ -802,30 +870,6 @@ __device__ __forceinline__ int cell_of_brick(const BatchCell *__restrict__ cells
   return lo;
 }
 
-// k_brick_list over the bricks of every cell of a batch (one wavefront per
-// brick); list entries are batch image indices.
-__global__ void __launch_bounds__(64) k_brick_list_batch(const BatchCell *__restrict__ cells, int ncell,
-                                                         const double4 *__restrict__ img,
-                                                         const double *__restrict__ rcut,
-                                                         uint32_t *__restrict__ cnt, const uint64_t *__restrict__ off,
-                                                         uint32_t *__restrict__ out) {
-  const uint32_t gb = blockIdx.x;
-  const BatchCell &C = cells[cell_of_brick(cells, ncell, gb)];
-  const Images I{img + C.img0, rcut, (int)C.nimg, C.brad};
-  const int b = (int)(gb - C.brick0);
-  const int lane = threadIdx.x;
-  uint32_t total = 0;
-  for (int m0 = 0; m0 < I.nimg; m0 += 64) {
-    const int m = m0 + lane;
-    const bool hit = (m < I.nimg) && image_hits_brick(C.G, I, b, m);
-    const uint64_t mask = __ballot(hit);
-    if (out && hit)
-      out[off[gb] + total + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull))] = C.img0 + (uint32_t)m;
-    total += (uint32_t)__popcll(mask);
-  }
-  if (!out && lane == 0) cnt[gb] = total;
-}
-
 __global__ void k_set_u32(uint32_t *p, uint32_t v) {
   if (blockIdx.x == 0 && threadIdx.x == 0) *p = v;
 }
@@ -835,10 +879,9 @@ __global__ void k_set_u32(uint32_t *p, uint32_t v) {
 // workgroup returns a brick number past the end, so all of them exit.
 __global__ void __launch_bounds__(256) k_promol_f_queue(const BatchCell *__restrict__ cells, int ncell,
                                                         uint32_t nbrick, PromolF T, const double4 *__restrict__ img,
-                                                        const float *__restrict__ cut2,
-                                                        const uint64_t *__restrict__ off,
-                                                        const uint32_t *__restrict__ lst, uint32_t *queue) {
+                                                        const double *__restrict__ rcut, uint32_t *queue) {
   __shared__ uint32_t next;
+  __shared__ ImageStage S;
   for (;;) {
     __syncthreads();  // every thread has read the previous brick number
     if (threadIdx.x == 0) next = atomicAdd(queue, 1u);
@@ -846,12 +889,8 @@ __global__ void __launch_bounds__(256) k_promol_f_queue(const BatchCell *__restr
     const uint32_t gb = next;
     if (gb >= nbrick) return;
     const BatchCell &C = cells[cell_of_brick(cells, ncell, gb)];
-    const int b = (int)(gb - C.brick0);
-    const int b1 = b % C.G.nb1, b2 = (b / C.G.nb1) % C.G.nb2, b3 = b / (C.G.nb1 * C.G.nb2);
-    const int t = threadIdx.x;
-    const int i = b1 * BX + (t % BX), j = b2 * BY + ((t / BX) % BY), k = b3 * BZ + t / (BX * BY);
-    if (i < C.G.n1 && j < C.G.n2 && k < C.G.n3)
-      promol_f_node(C.G, T, img, cut2, lst, off[gb], off[gb + 1], i, j, k, C.O);
+    const Images I{img + C.img0, rcut, (int)C.nimg, C.brad};
+    promol_brick<float>(C.G, T, I, (int)(gb - C.brick0), C.O, S);
   }
 }
 
@@ -891,7 +930,7 @@ void batch_nci_run(c2gpu_ctx *ctx, int ncell, const c2gpu_cell *cells, int nspec
     for (int a = 0; a < C.nat; a++)
       if (C.species[a] < 0 || C.species[a] >= nspecies) fail(C2GPU_ERR_ARG, "c2gpu_batch_run: bad species");
     BatchCell B;
-    B.G = make_geo(C.n, C.x2c);
+    B.G = make_geo(C.n, C.x2c, 1);
     std::vector<double> pos;
     std::vector<int> isp, iat;
     expand_images(C.x2c, C.nat, C.xat, C.species, rcmax, pos, isp, iat);
@@ -929,21 +968,6 @@ void batch_nci_run(c2gpu_ctx *ctx, int ncell, const c2gpu_cell *cells, int nspec
   double4 *d_img = buf<double4>(ctx, "bq_img", himg.size() > 0 ? himg.size() : 1);
   C2_HIP(hipMemcpyAsync(d_cells, hc.data(), sizeof(BatchCell) * hc.size(), hipMemcpyHostToDevice, st));
   C2_HIP(hipMemcpyAsync(d_img, himg.data(), sizeof(double4) * himg.size(), hipMemcpyHostToDevice, st));
-  uint32_t *cnt = buf<uint32_t>(ctx, "bq_bcnt", nbrick + 1);
-  uint64_t *off = buf<uint64_t>(ctx, "bq_boff", nbrick + 1);
-  C2_HIP(hipMemsetAsync(cnt + nbrick, 0, sizeof(uint32_t), st));
-  C2_LAUNCH(ctx, k_brick_list_batch, dim3((unsigned)nbrick), dim3(64), 0, d_cells, ncs, d_img, P.rcut, cnt,
-            (const uint64_t *)nullptr, (uint32_t *)nullptr);
-  size_t tmp = 0;
-  C2_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, cnt, off, (int)nbrick + 1, st));
-  void *t = buffer(ctx, "bq_bscan", tmp);
-  C2_HIP(hipcub::DeviceScan::ExclusiveSum(t, tmp, cnt, off, (int)nbrick + 1, st));
-  uint64_t total = 0;
-  copy_to_host(ctx, &total, off + nbrick, 8);
-  C2_HIP(hipStreamSynchronize(st));
-  uint32_t *lst = buf<uint32_t>(ctx, "bq_blst", total > 0 ? total : 1);
-  C2_LAUNCH(ctx, k_brick_list_batch, dim3((unsigned)nbrick), dim3(64), 0, d_cells, ncs, d_img, P.rcut, cnt, off,
-            lst);
   uint32_t *queue = buf<uint32_t>(ctx, "bq_queue", 1);
   int ncu = 256;
   (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, ctx->device);
@@ -955,8 +979,7 @@ void batch_nci_run(c2gpu_ctx *ctx, int ncell, const c2gpu_cell *cells, int nspec
     C2_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
     hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(64), 0, st, queue, 0u);  // no memset nodes in graphs
     hipLaunchKernelGGL(k_promol_f_queue, dim3(nwg), dim3(256), 0, st, d_cells, ncs, (uint32_t)nbrick, P.F,
-                       (const double4 *)d_img, (const float *)P.cut2f, (const uint64_t *)off,
-                       (const uint32_t *)lst, queue);
+                       (const double4 *)d_img, (const double *)P.rcut, queue);
     C2_HIP(hipStreamEndCapture(st, &g));
     C2_HIP(hipGetLastError());
     C2_HIP(hipGraphInstantiate(&ge, g, nullptr, nullptr, 0));
@@ -1013,7 +1036,7 @@ void nci_run(c2gpu_ctx *ctx, const double *rho, const int n[3], const double x2c
     if (n[c] < 1) fail(C2GPU_ERR_ARG, "c2gpu_nci: bad grid");
   const size_t N = (size_t)n[0] * n[1] * n[2];
   hipStream_t st = ctx->stream;
-  const Geo G = make_geo(n, x2c);
+  const Geo G = make_geo(n, x2c, scheme == C2GPU_NCI_PROMOL && zfast);
   const size_t osz = out_f32 ? 4 : 8;
   const bool dev = flags & C2GPU_PTR_DEVICE;
   NciOut O;
@@ -1024,12 +1047,12 @@ void nci_run(c2gpu_ctx *ctx, const double *rho, const int n[3], const double x2c
   const unsigned g = grid_for((int64_t)N, 256);
   if (scheme == C2GPU_NCI_PROMOL) {
     PromolDev P = upload_promol(ctx, promol, x2c);
-    BrickLists BL = build_bricks(ctx, G, P.img, P.rcut, P.nimg, "pm");
+    const Images I{P.img, P.rcut, P.nimg, brick_radius(G)};
     const int nbk = G.nb1 * G.nb2 * G.nb3;
     if (precision == C2GPU_FP32)
-      C2_LAUNCH(ctx, k_promol_f, dim3(nbk), dim3(256), 0, G, P.F, P.img, P.cut2f, BL.off, BL.lst, O);
+      C2_LAUNCH(ctx, k_promol_f, dim3(nbk), dim3(256), 0, G, P.F, I, O);
     else
-      C2_LAUNCH(ctx, k_promol_d, dim3(nbk), dim3(256), 0, G, P.D, P.img, BL.off, BL.lst, O);
+      C2_LAUNCH(ctx, k_promol_d, dim3(nbk), dim3(256), 0, G, P.D, I, O);
   } else if (scheme == C2GPU_NCI_FFT) {
     if (precision != C2GPU_FP64) fail(C2GPU_ERR_UNSUPPORTED, "c2gpu_nci: FFT scheme runs in FP64");
     const double *d_rho = to_device_grid(ctx, rho, N, flags, "nci_rho");
@@ -1137,7 +1160,7 @@ void nci_promol_nodes_run(c2gpu_ctx *ctx, const c2gpu_nci_nodes *nd, const doubl
   double lo[3], hi[3];
   box_frac_range(G, x2c, lo, hi);
   PromolDev P = upload_promol(ctx, pm, x2c, lo, hi);
-  BrickLists BL = build_bricks(ctx, G, P.img, P.rcut, P.nimg, "pm");
+  const Images I{P.img, P.rcut, P.nimg, brick_radius(G)};
   NciOut O;
   O.is_f32 = f32 ? 1 : 0;
   O.zfast = 1;
@@ -1146,9 +1169,9 @@ void nci_promol_nodes_run(c2gpu_ctx *ctx, const c2gpu_nci_nodes *nd, const doubl
   O.rhoat = rhoat_out ? (dev ? rhoat_out : buffer(ctx, "nci_rhoat", osz * N)) : nullptr;
   const int nbk = G.nb1 * G.nb2 * G.nb3;
   if (f32)
-    C2_LAUNCH(ctx, k_promol_f, dim3(nbk), dim3(256), 0, G, P.F, P.img, P.cut2f, BL.off, BL.lst, O);
+    C2_LAUNCH(ctx, k_promol_f, dim3(nbk), dim3(256), 0, G, P.F, I, O);
   else
-    C2_LAUNCH(ctx, k_promol_d, dim3(nbk), dim3(256), 0, G, P.D, P.img, BL.off, BL.lst, O);
+    C2_LAUNCH(ctx, k_promol_d, dim3(nbk), dim3(256), 0, G, P.D, I, O);
   if (!dev) {
     copy_out(ctx, crho_out, O.crho, osz * N);
     copy_out(ctx, cgrad_out, O.cgrad, osz * N);

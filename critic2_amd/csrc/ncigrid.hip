@@ -74,11 +74,8 @@ __device__ __forceinline__ void hermite_cr(double u, double w[4], double d[4], d
 
 __global__ void __launch_bounds__(256) k_nci_grid(Geo G, GridInterp T, const double *__restrict__ rho,
                                                   NciOut O) {
-  const int b = blockIdx.x;
-  const int b1 = b % G.nb1, b2 = (b / G.nb1) % G.nb2, b3 = b / (G.nb1 * G.nb2);
-  const int t = threadIdx.x;
-  const int i = b1 * BX + (t % BX), j = b2 * BY + ((t / BX) % BY), k = b3 * BZ + t / (BX * BY);
-  if (i >= G.n1 || j >= G.n2 || k >= G.n3) return;
+  int i, j, k;
+  if (!brick_node(G, blockIdx.x, threadIdx.x, i, j, k)) return;
   double wx[3];
   grid_node_frac(T, i, j, k, wx);
   const int nn[3] = {G.n1, G.n2, G.n3};
