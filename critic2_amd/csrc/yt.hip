@@ -20,7 +20,7 @@
 //                 maxima); equal means the point's basin (a point joins a
 //                 basin exactly when every upward path ends in it),
 //                 different means a surface point;
-//   k_yt_w_narrow / k_yt_w_wide_step
+//   k_yt_w_dense (up to DENSE_MAX attractors), k_yt_w_narrow / k_yt_w_wide_step
 //                 the surface points' weights, a sparse vector of basins
 //                 each (16 lanes per point up to 32 basins, a workgroup
 //                 beyond), in the same topological order over the surface
@@ -59,6 +59,7 @@ constexpr double VSMALL = 1e-40;  // param.F90 vsmall
 struct YtGeo {
   int n1, n2, n3, nvec;
   int di[14], dj[14], dk[14];
+  int op[14];  // the facet across: -(di, dj, dk)
   double al[14];
   // the reference sort's rank of every point (qcksort_order), set when the
   // grid has equal values where the order matters; else null and values
@@ -76,6 +77,7 @@ __device__ __forceinline__ double yt_key(const YtGeo &G, const double *__restric
 }
 
 __device__ __forceinline__ int wrapn(int x, int n) {
+  if ((unsigned)x < (unsigned)n) return x;  // no division but at the cell's faces
   x %= n;
   return x < 0 ? x + n : x;
 }
@@ -169,34 +171,58 @@ __device__ __forceinline__ uint64_t yt_lohi_of(const YtGeo &G, uint32_t p, const
   return ((uint64_t)lo << 32) | hi;
 }
 
+// Appends val where pred holds, one atomic per workgroup: with one per
+// wavefront the counter's address took thousands of atomics a frontier, one
+// after the other.  Every thread calls it, with the same two LDS words.
+__device__ __forceinline__ void yt_append_block(bool pred, uint32_t val, uint32_t *list, uint32_t *n, uint32_t *cnt,
+                                                uint32_t *base) {
+  if (threadIdx.x == 0) *cnt = 0;
+  __syncthreads();
+  uint32_t at = 0;
+  if (pred) at = atomicAdd(cnt, 1u);
+  __syncthreads();
+  if (threadIdx.x == 0 && *cnt) *base = atomicAdd(n, *cnt);
+  __syncthreads();
+  if (pred) list[*base + at] = val;
+}
+
+// Whether p is the last pending higher neighbour of its neighbour across
+// facet q (jn): jn's own mask says whether p is above it, so no densities
+// are read.
+__device__ __forceinline__ bool yt_release(const YtGeo &G, uint32_t p, int q, const uint16_t *__restrict__ hmask,
+                                           const int32_t *__restrict__ lab, uint32_t *__restrict__ pend,
+                                           uint32_t &jn) {
+  int i, j, k;
+  coords3(G, p, i, j, k);
+  jn = nbr(G, i, j, k, q);
+  return ((hmask[jn] >> G.op[q]) & 1) && (!lab || lab[jn] == 0) && atomicSub(&pend[jn], 1u) == 1u;
+}
+
 // One frontier of the labels: every point of `front` is final; each lower
 // neighbour loses one pending higher neighbour, and the thread that takes
 // the last computes it and puts it on the next frontier.
 // (The frontier's size is read from nfp, written by the step before, so the
 // host need not read it back between frontiers; a grid-stride loop covers
 // it, and an empty frontier makes the launch a no-op.)
+// A frontier holds about 10^4 points and a launch is all latency, so each
+// facet of a point is a thread of its own (LN threads a point): one chain of
+// mask, atomic, neighbours' labels and append, where a thread per point walked
+// its 6 to 14 facets one after the other.  200x192x240, 864 frontiers: 30.5 ->
+// 13.4 us a launch.
+template <int LN>
 __global__ void __launch_bounds__(YB) k_yt_lab_step(YtGeo G, const uint32_t *nfp, const uint32_t *__restrict__ front,
-                                                     const double *__restrict__ g,
                                                      const uint16_t *__restrict__ hmask, uint32_t *__restrict__ pend,
                                                      uint64_t *lohi, uint32_t *__restrict__ next, uint32_t *nnext) {
-  const uint32_t nf = *nfp;
-  for (uint32_t b0 = blockIdx.x * YB; b0 < nf; b0 += gridDim.x * YB) {  // uniform per workgroup
-    const uint32_t t = b0 + threadIdx.x;
-    uint32_t done[14];
-    int nd = 0;
-    if (t < nf) {
-      const uint32_t p = front[t];
-      int i, j, k;
-      coords3(G, p, i, j, k);
-      for (int q = 0; q < G.nvec; q++) {
-        const uint32_t jn = nbr(G, i, j, k, q);
-        if (yt_above(G, g, p, jn) && atomicSub(&pend[jn], 1u) == 1u) {
-          lohi[jn] = yt_lohi_of(G, jn, hmask, lohi);
-          done[nd++] = jn;
-        }
-      }
-    }
-    for (int q = 0; q < 14; q++) yt_append(q < nd, q < nd ? done[q] : 0u, next, nnext);
+  __shared__ uint32_t cnt, base;
+  const uint64_t nl = (uint64_t)*nfp * LN;
+  for (uint64_t b0 = (uint64_t)blockIdx.x * YB; b0 < nl; b0 += (uint64_t)gridDim.x * YB) {  // uniform per workgroup
+    const uint64_t l = b0 + threadIdx.x;
+    const int q = (int)(l % LN);
+    uint32_t jn = 0;
+    const bool last = l < nl && q < G.nvec && yt_release(G, front[l / LN], q, hmask, nullptr, pend, jn);
+    if (last) lohi[jn] = yt_lohi_of(G, jn, hmask, lohi);
+    yt_append_block(last, jn, next, nnext, &cnt, &base);
+    __syncthreads();
   }
 }
 
@@ -521,6 +547,182 @@ __global__ void __launch_bounds__(YB) k_yt_w_wide_step(YtGeo G, const uint32_t *
   }
 }
 
+// One frontier of the weights in one launch, for cells of at most DENSE_MAX
+// attractors: GL lanes a point, a dense accumulator per basin and point in
+// LDS.  Lane a takes the point's a-th higher neighbour in facet order (its
+// fraction, formed as yt_fracs forms it, and its rank in decreasing rho); the
+// neighbours are then added in rank order, each neighbour's entries by the
+// lanes at once (its basins are distinct), so every basin's weight adds the
+// contributions in the order of yt_weights.  All neighbours' first GL entries
+// are loaded before any is added.  The basins present leave in increasing
+// order, with pool room for the whole workgroup by one atomic; then the next
+// frontier: each surface point below a frontier point loses one pending
+// neighbour, and the thread that takes the last lists it.
+// A frontier holds about 6000 points and is all latency: merging the sorted
+// lists basin by basin (k_yt_w_narrow) waited for a load per basin, and points
+// of more than KW basins for a launch of their own.  200x192x240, 74 atoms,
+// 824 frontiers: 44 us, 25 us for the wide points and the next frontier and a
+// memset before; 23.6 us now.
+constexpr int DENSE_MAX = 416;  // 9 bytes x YB / GL points of LDS each: below 60 KiB
+struct NbrRec {
+  uint64_t so;  // its entries
+  double fr;    // its fraction
+  int32_t lab;  // its basin (interior), or 0
+  int32_t len;
+};
+__global__ void __launch_bounds__(YB) k_yt_w_dense(YtGeo G, const uint32_t *nfp, const uint32_t *__restrict__ front,
+                                                    const double *__restrict__ g, const uint16_t *__restrict__ hmask,
+                                                    const int32_t *__restrict__ lab, const int32_t *__restrict__ slot,
+                                                    WBuf W, int nattr, unsigned long long *widetot, int *err,
+                                                    uint32_t *__restrict__ pend, uint32_t *__restrict__ next,
+                                                    uint32_t *nnext) {
+  constexpr int PB = YB / GL;
+  extern __shared__ double dacc[];  // PB x nattr doubles, then PB x nattr flags
+  __shared__ NbrRec rec[PB][14];
+  __shared__ uint32_t cnt, cbase, want[PB], nwide;
+  __shared__ unsigned long long top;
+  const uint32_t nf = *nfp;
+  const int gi = threadIdx.x / GL, r = threadIdx.x % GL;
+  double *acc = dacc + (size_t)gi * nattr;
+  uint8_t *pres = reinterpret_cast<uint8_t *>(dacc + (size_t)PB * nattr) + (size_t)gi * nattr;
+  const int seg = (nattr + GL - 1) / GL, s0 = r * seg < nattr ? r * seg : nattr, s1 = s0 + seg < nattr ? s0 + seg : nattr;
+  for (uint32_t b0 = blockIdx.x * PB; b0 < nf; b0 += gridDim.x * PB) {  // uniform per workgroup
+    const bool in = b0 + gi < nf;
+    if (threadIdx.x == 0) nwide = 0;
+    uint32_t p = 0, mine = 0;
+    int nh = 0;
+    if (in) {  // whole groups
+      p = front[b0 + gi];
+      for (int a = r; a < nattr; a += GL) {
+        acc[a] = 0.0;
+        pres[a] = 0;
+      }
+      int i, j, k;
+      coords3(G, p, i, j, k);
+      const double gp = g[p];
+      const uint32_t mask = hmask[p];
+      nh = __popc(mask);
+      int q = -1;  // the r-th set bit of the mask
+      for (int u = 0, c = 0; u < G.nvec; u++)
+        if (mask & (1u << u)) {
+          if (c == r) q = u;
+          c++;
+        }
+      double chi = 0.0, kj = 0.0;
+      NbrRec N{0, 0.0, 0, 0};
+      if (q >= 0) {
+        const uint32_t jn = nbr(G, i, j, k, q);
+        const double gj = g[jn];
+        N.lab = lab[jn];
+        const int32_t sj = slot[jn];  // meaningless for an interior neighbour
+        kj = yt_key(G, g, jn);
+        chi = fmax(G.al[q] * (gj - gp), VSMALL);
+        N.len = 1;
+        if (N.lab == 0) {
+          N.len = W.c[sj];
+          N.so = W.off[sj];
+        }
+      }
+      double csum = 0.0;
+      for (int u = 0; u < nh; u++) csum = csum + __shfl(chi, u, GL);
+      N.fr = chi / fmax(csum, VSMALL);
+      int rank = 0;
+      for (int u = 0; u < nh; u++) {
+        const double ku = __shfl(kj, u, GL);
+        rank += (ku > kj || (ku == kj && u < r)) ? 1 : 0;
+      }
+      if (q >= 0) rec[gi][rank] = N;
+    }
+    __syncthreads();
+    if (in) {
+      uint32_t pb[14];
+      double pw[14];
+#pragma unroll
+      for (int kk = 0; kk < 14; kk++) {
+        pb[kk] = 0;
+        pw[kk] = 1.0;
+        if (kk < nh) {
+          const NbrRec N = rec[gi][kk];
+          if (N.lab != 0) {
+            pb[kk] = r == 0 ? (uint32_t)N.lab : 0u;
+          } else if (r < N.len) {
+            pb[kk] = W.b[N.so + r];
+            pw[kk] = W.w[N.so + r];
+          }
+        }
+      }
+#pragma unroll
+      for (int kk = 0; kk < 14; kk++) {
+        if (kk < nh) {
+          const double fr = rec[gi][kk].fr;
+          if (pb[kk]) {
+            acc[pb[kk] - 1] = acc[pb[kk] - 1] + fr * pw[kk];
+            pres[pb[kk] - 1] = 1;
+          }
+          if (rec[gi][kk].lab == 0)
+            for (int e = r + GL; e < rec[gi][kk].len; e += GL) {
+              const uint32_t b = W.b[rec[gi][kk].so + e];
+              acc[b - 1] = acc[b - 1] + fr * W.w[rec[gi][kk].so + e];
+              pres[b - 1] = 1;
+            }
+        }
+        __builtin_amdgcn_wave_barrier();  // the next neighbour reads what this one's lanes wrote
+      }
+      for (int a = s0; a < s1; a++) mine += pres[a];
+    }
+    // the lanes' segments of the basins, in order
+    uint32_t incl = mine;
+    for (int o = 1; o < GL; o <<= 1) {
+      const uint32_t v = __shfl_up(incl, o, GL);
+      if (r >= o) incl += v;
+    }
+    const uint32_t nb = __shfl(incl, GL - 1, GL);
+    if (r == 0) {
+      want[gi] = nb;
+      if (nb > KW) atomicAdd(&nwide, 1u);
+    }
+    __syncthreads();
+    uint32_t before = 0, all = 0;
+#pragma unroll
+    for (int u = 0; u < PB; u++) {
+      const uint32_t v = want[u];
+      before += u < gi ? v : 0u;
+      all += v;
+    }
+    if (threadIdx.x == 0) {
+      if (all) top = atomicAdd(W.top, (unsigned long long)all);
+      if (nwide) atomicAdd(widetot, (unsigned long long)nwide);
+    }
+    uint32_t jn = 0;
+    const bool last = in && r < G.nvec && yt_release(G, p, r, hmask, lab, pend, jn);
+    yt_append_block(last, jn, next, nnext, &cnt, &cbase);  // its barriers publish top
+    if (in) {
+      const uint32_t t = (uint32_t)slot[p];
+      unsigned long long o = top + before;
+      if (o + (unsigned long long)nb > W.cap) {  // pool full: the host enlarges it and runs the weights again
+        if (r == 0) {
+          atomicOr(err, 4);
+          W.c[t] = 0;
+          W.off[t] = 0;
+        }
+      } else {
+        if (r == 0) {
+          W.c[t] = (uint16_t)nb;
+          W.off[t] = o;
+        }
+        o += incl - mine;
+        for (int a = s0; a < s1; a++)
+          if (pres[a]) {
+            W.b[o] = (uint32_t)(a + 1);
+            W.w[o] = acc[a];
+            o++;
+          }
+      }
+    }
+    __syncthreads();
+  }
+}
+
 // Pending surface neighbours above each surface point; those with none
 // form the first frontier.
 __global__ void __launch_bounds__(YB) k_yt_w_init(YtGeo G, uint32_t nias, const uint32_t *__restrict__ ias,
@@ -674,6 +876,12 @@ void yt_run(c2gpu_ctx *ctx, const double *rho, const int n[3], const double x2c[
     G.dj[q] = vec[3 * q + 1];
     G.dk[q] = vec[3 * q + 2];
   }
+  for (int q = 0; q < G.nvec; q++) {
+    G.op[q] = -1;
+    for (int u = 0; u < G.nvec; u++)
+      if (G.di[u] == -G.di[q] && G.dj[u] == -G.dj[q] && G.dk[u] == -G.dk[q]) G.op[q] = u;
+    if (G.op[q] < 0) fail(C2GPU_ERR_ARG, "c2gpu_yt: internal inconsistency in the grid lattice's facets");
+  }
   // inputs on the device
   const double *g = rho;
   YtFields F{};
@@ -701,7 +909,8 @@ void yt_run(c2gpu_ctx *ctx, const double *rho, const int n[3], const double x2c[
   C2_HIP(hipMemsetAsync(d_cnt, 0, 8, st));
   C2_HIP(hipMemsetAsync(d_err, 0, 8, st));
   const unsigned gN = grid_for(N, YB);
-  const unsigned gF = (unsigned)persistent_threads(ctx->device, YB) / YB;  // frontier kernels, grid-stride
+  // frontier kernels, grid-stride: 4 workgroups a CU (frontiers are short)
+  const unsigned gF = (unsigned)persistent_threads(ctx->device, YB) / YB / 2;
   uint32_t *pend = buf<uint32_t>(ctx, "yt_pend", N);
   C2_LAUNCH(ctx, k_yt_class, dim3(gN), dim3(YB), 0, G, N, g, hmask, pend, maxl, d_cnt, d_err);
   add_kernel_bytes(ctx, "k_yt_class", (double)N * (8.0 * (G.nvec + 1) + 2.0));
@@ -788,13 +997,18 @@ void yt_run(c2gpu_ctx *ctx, const double *rho, const int n[3], const double x2c[
   for (;;) {
     fc.reserve(passes + FRONT_BATCH + 1);
     for (int u = 0; u < FRONT_BATCH; u++, passes++)
-      C2_LAUNCH(ctx, k_yt_lab_step, dim3(gF), dim3(YB), 0, G, fc.at(passes), fr[passes & 1], g, hmask, pend, lohi,
-                fr[(passes & 1) ^ 1], fc.at(passes + 1));
+      if (G.nvec <= 8)
+        C2_LAUNCH(ctx, k_yt_lab_step<8>, dim3(gF), dim3(YB), 0, G, fc.at(passes), fr[passes & 1], hmask, pend, lohi,
+                  fr[(passes & 1) ^ 1], fc.at(passes + 1));
+      else
+        C2_LAUNCH(ctx, k_yt_lab_step<16>, dim3(gF), dim3(YB), 0, G, fc.at(passes), fr[passes & 1], hmask, pend, lohi,
+                  fr[(passes & 1) ^ 1], fc.at(passes + 1));
     if (read_scalar(ctx, fc.at(passes)) == 0) break;
   }
   uint64_t ndone = 0;
   passes = fc.finish(passes, ndone);
-  add_kernel_bytes(ctx, "k_yt_lab_step", (double)ndone * (4.0 + 8.0 * G.nvec * 2.0));
+  add_kernel_bytes(ctx, G.nvec <= 8 ? "k_yt_lab_step<8>" : "k_yt_lab_step<16>",
+                   (double)ndone * (4.0 + 8.0 * G.nvec * 2.0));
   if (ndone != N) fail(C2GPU_ERR_ARG, "c2gpu_yt: internal inconsistency in the label order");
   S.label_passes = passes;
   int32_t *lab = dev && label_out ? label_out : buf<int32_t>(ctx, "yt_lab", N);
@@ -813,7 +1027,7 @@ void yt_run(c2gpu_ctx *ctx, const double *rho, const int n[3], const double x2c[
     W.off = buf<uint64_t>(ctx, "yt_woff", nias);
     W.c = buf<uint16_t>(ctx, "yt_wc", nias);
     W.top = buf<unsigned long long>(ctx, "yt_wtop", 1);
-    uint32_t *wide = buf<uint32_t>(ctx, "yt_wide", nias);
+    uint32_t *wide = nattr > DENSE_MAX ? buf<uint32_t>(ctx, "yt_wide", nias) : nullptr;
     unsigned long long *widetot = buf<unsigned long long>(ctx, "yt_widetot", 1);
     const size_t wide_lds = 9 * (size_t)nattr;
     if (wide_lds > 120 * 1024) fail(C2GPU_ERR_UNSUPPORTED, "c2gpu_yt: too many attractors for the LDS accumulator");
@@ -834,6 +1048,12 @@ void yt_run(c2gpu_ctx *ctx, const double *rho, const int n[3], const double x2c[
         wc.reserve(wpasses + FRONT_BATCH + 1);
         for (int u = 0; u < FRONT_BATCH; u++, wpasses++) {
           uint32_t *cf = fr[wpasses & 1], *nx = fr[(wpasses & 1) ^ 1];
+          if (nattr <= DENSE_MAX) {
+            C2_LAUNCH(ctx, k_yt_w_dense, dim3(gF), dim3(YB), 9 * (size_t)nattr * (YB / GL), G,
+                      (const uint32_t *)wc.at(wpasses), cf, g, hmask, lab, slot, W, nattr, widetot, d_err, pend, nx,
+                      wc.at(wpasses + 1));
+            continue;
+          }
           C2_HIP(hipMemsetAsync(d_cnt, 0, 4, st));  // the frontier's wide points
           C2_LAUNCH(ctx, k_yt_w_narrow, dim3(gF), dim3(YB), 0, G, wc.at(wpasses), cf, g, hmask, lab, slot, W, wide,
                     d_cnt, widetot, d_err);
@@ -847,10 +1067,11 @@ void yt_run(c2gpu_ctx *ctx, const double *rho, const int n[3], const double x2c[
       wpasses = wc.finish(wpasses, wdone);
       S.wide = (int)read_scalar(ctx, widetot);
       // each point: its and its higher neighbours' rho, masks, labels and slots
-      add_kernel_bytes(ctx, "k_yt_w_narrow", (double)wdone * (4.0 + 2.0 + 8.0 * (G.nvec + 1) + 8.0 * G.nvec));
+      const char *wk = nattr <= DENSE_MAX ? "k_yt_w_dense" : "k_yt_w_narrow";
+      add_kernel_bytes(ctx, wk, (double)wdone * (4.0 + 2.0 + 8.0 * (G.nvec + 1) + 8.0 * G.nvec));
       if (wdone != nias) fail(C2GPU_ERR_ARG, "c2gpu_yt: internal inconsistency in the weight order");
       // weight entries: each written once and read back by the points below
-      add_kernel_bytes(ctx, "k_yt_w_narrow", 24.0 * (double)read_scalar(ctx, W.top));
+      add_kernel_bytes(ctx, wk, 24.0 * (double)read_scalar(ctx, W.top));
       const int e = read_scalar(ctx, d_err);
       if (!(e & 4)) break;
       cap = read_scalar(ctx, W.top) + (cap >> 1);  // every entry asked for, and room to spare

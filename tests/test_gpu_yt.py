@@ -164,3 +164,23 @@ def test_yt_edge_grids(ctx, name, seed, edge, ang, nat, n):
     assert int(np.count_nonzero(got["labels"] != idg)) == 0
     np.testing.assert_allclose(got["vol"], vol, rtol=1e-10)
     np.testing.assert_allclose(got["sums"], sums, rtol=1e-10)
+
+
+@pytest.mark.parametrize("ang", [(90, 90, 90), (80, 100, 105)])
+def test_yt_weights_either_side_of_the_dense_limit(ctx, ang):
+    """The accumulators of up to 416 attractors in LDS and the list merge
+    beyond: known points that no maximum takes pad the attractor count, and
+    leave labels, weights and sums as they are without them."""
+    cell = random_cell(67, (8.0, 8.5, 9.0), ang, 30, (1, 6, 7, 8), (30, 33, 35))
+    f = gb.synth_slater(ctx, cell)
+    ref, got = _run_both(ctx, cell, f, {})
+    np.testing.assert_allclose(got["vol"], ref[3], rtol=1e-10)
+    for total in (415, 416, 417):
+        print(f"[case] yt dense limit {total} {ang}", flush=True)
+        cps = np.random.default_rng(total).uniform(size=(total - 30, 3))
+        r = gy.yt_integrate(ctx, f, cell.n, cell.x2c, cell.xat, fields=[f, f * f], cps=cps)
+        assert r["nattr"] == total
+        np.testing.assert_array_equal(r["labels"], ref[0])
+        np.testing.assert_allclose(r["vol"][:30], ref[3], rtol=1e-10)
+        np.testing.assert_allclose(r["sums"][:, :30], ref[4], rtol=1e-10)
+        assert not r["vol"][30:].any()
