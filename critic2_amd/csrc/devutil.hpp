@@ -10,6 +10,16 @@
 
 namespace c2 {
 
+// The 8 XCDs take workgroups in turn, each with an L2 of its own: workgroup b
+// of a launch works on slice xcd_block<R>() of the data, so that an XCD takes
+// R neighbouring slices while all of them stay within 8 R.  A permutation of
+// 0..gridDim.x-1.
+template <uint32_t R>
+__device__ __forceinline__ uint32_t xcd_block() {
+  const uint32_t b = blockIdx.x, g = b / (8 * R) * (8 * R), q = b - g;
+  return g + 8 * R <= gridDim.x ? g + (q & 7u) * R + (q >> 3) : b;
+}
+
 struct Timer {
   hipStream_t s;
   hipEvent_t a, b;
