@@ -142,20 +142,69 @@ struct RadTabD {  // FP64 tables, exact grid1%interp
 struct PromolD {
   const double *r, *f, *fp, *fpp;  // concatenated tables
   // 1/(r_i - r_j), j < i, of the four nodes from r on: (1,0) (2,0) (2,1)
-  // (3,0) (3,1) (3,2), six per node (k_table_inv)
+  // (3,0) (3,1) (3,2), six per node (k_table_build)
   const double *inv;
   const int *toff, *tng;           // per species offset / ngrid
   const double *ta, *tb, *trmax, *tcut;
 };
 
-// The reciprocal node differences of interp_d, once per call instead of six
-// divisions per atom and node: the same quotients.  Entries whose four nodes
-// run past their table are never read.
-__global__ void k_table_inv(int n, const double *__restrict__ r, double *__restrict__ inv) {
+// What the evaluators read beside the tables themselves, once per call, one
+// thread per node q of the concatenated tables: the reciprocal differences of
+// the four nodes from q on (interp_d: six divisions per atom and node
+// otherwise, the same quotients), and, for base = q's index in its table, the
+// FP32 cubics of the interval's 4-node Lagrange interpolants in u = r -
+// r(base-1), with the node.  Built on the host before and copied table by
+// table: 0.2 ms of every call.  Contraction is off: the coefficients are those
+// of separate products and sums.
+__global__ void __launch_bounds__(64) k_table_build(int tot, int ns, const double *__restrict__ r,
+                                                    const double *__restrict__ f, const double *__restrict__ fp,
+                                                    const double *__restrict__ fpp, const int *__restrict__ toff,
+                                                    const int *__restrict__ tng, double *__restrict__ inv,
+                                                    float *__restrict__ coef, float *__restrict__ node) {
+#pragma clang fp contract(off)
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= n) return;
-  for (int i = 1, e = 0; i < 4; i++)
-    for (int j = 0; j < i; j++, e++) inv[6 * (size_t)q + e] = q + 3 < n ? 1.0 / (r[q + i] - r[q + j]) : 0.0;
+  if (q >= tot) return;
+  for (int i = 1, e = 0; i < 4; i++)  // entries past their table are never read
+    for (int j = 0; j < i; j++, e++) inv[6 * (size_t)q + e] = q + 3 < tot ? 1.0 / (r[q + i] - r[q + j]) : 0.0;
+  int s = 0;
+  while (s + 1 < ns && toff[s + 1] <= q) s++;
+  const int base = q - toff[s];
+  float c[16];
+  for (int d = 0; d < 16; d++) c[d] = 0.f;
+  float nd = 0.f;
+  if (base >= 2 && base <= tng[s] - 2) {
+    double rr[4];
+    for (int i = 0; i < 4; i++) rr[i] = r[q - 2 + i];
+    const double u0 = rr[1];
+    double pc[3][4] = {{0}};
+    for (int i = 0; i < 4; i++) {
+      // the polynomial prod_{j != i} (u - (r_j - u0)) / (r_i - r_j)
+      double poly[4] = {1, 0, 0, 0};
+      double den = 1;
+      for (int j = 0; j < 4; j++) {
+        if (j == i) continue;
+        const double root = rr[j] - u0;
+        double np[4] = {0, 0, 0, 0};
+        for (int d = 0; d < 3; d++) {
+          np[d + 1] += poly[d];
+          np[d] -= root * poly[d];
+        }
+        for (int d = 0; d < 4; d++) poly[d] = np[d];
+        den *= (rr[i] - rr[j]);
+      }
+      const int ii = q - 2 + i;
+      for (int d = 0; d < 4; d++) {
+        pc[0][d] += f[ii] * poly[d] / den;
+        pc[1][d] += fp[ii] * poly[d] / den;
+        pc[2][d] += fpp[ii] * poly[d] / den;
+      }
+    }
+    for (int t = 0; t < 3; t++)
+      for (int d = 0; d < 4; d++) c[4 * t + d] = (float)pc[t][d];
+    nd = (float)u0;
+  }
+  for (int d = 0; d < 16; d++) coef[(size_t)q * 16 + d] = c[d];
+  node[q] = nd;
 }
 
 // grid1%interp (grid1mod@proc.f90:86-137), FP64, same operation order
@@ -540,22 +589,26 @@ static void expand_images(const double x2c[9], int nat, const double *xat, const
     tlo[c] = (int)std::floor(flo[c] - delta[c]) - 1;
     thi[c] = (int)std::ceil(fhi[c] + delta[c]) + 1;
   }
-  for (int at = 0; at < nat; at++)
-    for (int t0 = tlo[0]; t0 <= thi[0]; t0++)
-      for (int t1 = tlo[1]; t1 <= thi[1]; t1++)
+  for (int at = 0; at < nat; at++) {
+    double x0[3];
+    for (int c = 0; c < 3; c++) x0[c] = xat[3 * at + c] - std::floor(xat[3 * at + c]);
+    auto out = [&](int c, double v) { return v < flo[c] - delta[c] || v > fhi[c] + delta[c]; };
+    for (int t0 = tlo[0]; t0 <= thi[0]; t0++) {
+      const double f0 = x0[0] + t0;
+      if (out(0, f0)) continue;
+      for (int t1 = tlo[1]; t1 <= thi[1]; t1++) {
+        const double f1 = x0[1] + t1;
+        if (out(1, f1)) continue;
         for (int t2 = tlo[2]; t2 <= thi[2]; t2++) {
-          double xf[3] = {xat[3 * at] - std::floor(xat[3 * at]) + t0,
-                          xat[3 * at + 1] - std::floor(xat[3 * at + 1]) + t1,
-                          xat[3 * at + 2] - std::floor(xat[3 * at + 2]) + t2};
-          bool ok = true;
-          for (int c = 0; c < 3; c++)
-            if (xf[c] < flo[c] - delta[c] || xf[c] > fhi[c] + delta[c]) ok = false;
-          if (!ok) continue;
-          for (int r = 0; r < 3; r++)
-            pos.push_back(x2c[r] * xf[0] + x2c[r + 3] * xf[1] + x2c[r + 6] * xf[2]);
+          const double f2 = x0[2] + t2;
+          if (out(2, f2)) continue;
+          for (int r = 0; r < 3; r++) pos.push_back(x2c[r] * f0 + x2c[r + 3] * f1 + x2c[r + 6] * f2);
           isp.push_back(spc[at]);
           iat.push_back(at);
         }
+      }
+    }
+  }
 }
 
 struct BrickLists {
@@ -625,116 +678,90 @@ void synth_slater_run(c2gpu_ctx *ctx, const double x2c[9], const int n[3], int n
 struct PromolDev {
   PromolD D;
   PromolF F;
-  double4 *img;
-  double *rcut;
+  const double4 *img;
+  const double *rcut;
   int nimg;
 };
 
-// The radial tables on the device (FP64 nodes and values, FP32 cubic
-// coefficients); returns the largest cutoff min(cutrad, rmax).
-static double upload_tables(c2gpu_ctx *ctx, int ns, const c2gpu_radial_table *tables, PromolDev &P) {
+// The largest cutoff min(cutrad, rmax) of the tables (list_near_atoms'
+// up2dsp, crystalmod@env.f90:676-690); checks them.
+static double table_reach(int ns, const c2gpu_radial_table *tables) {
   if (ns < 1 || !tables) fail(C2GPU_ERR_ARG, "c2gpu_nci: radial tables required");
-  std::vector<int> toff(ns), tng(ns);
-  int tot = 0;
   double rcmax = 0;
-  std::vector<double> ta(ns), tb(ns), trmax(ns), tcut(ns);
   for (int s = 0; s < ns; s++) {
     const c2gpu_radial_table &t = tables[s];
     if (t.ngrid < 6 || !t.r || !t.f || !t.fp || !t.fpp) fail(C2GPU_ERR_ARG, "c2gpu_nci: bad radial table");
-    toff[s] = tot;
-    tng[s] = t.ngrid;
-    tot += t.ngrid;
-    ta[s] = t.a;
-    tb[s] = t.b;
-    trmax[s] = t.rmax;
-    // list_near_atoms up2dsp = min(cutrad, rmax), crystalmod@env.f90:676-690
-    tcut[s] = t.cutrad < t.rmax ? t.cutrad : t.rmax;
-    rcmax = tcut[s] > rcmax ? tcut[s] : rcmax;
+    const double rc = t.cutrad < t.rmax ? t.cutrad : t.rmax;
+    rcmax = rc > rcmax ? rc : rcmax;
   }
-  std::vector<double> r(tot), f(tot), fp(tot), fpp(tot);
-  for (int s = 0; s < ns; s++) {
+  return rcmax;
+}
+
+// The checked radial tables and the atoms `img` (position, species) on the
+// device: one copy from the pinned staging buffer, and the derived tables
+// built there.
+static PromolDev upload_tables(c2gpu_ctx *ctx, int ns, const c2gpu_radial_table *tables,
+                               const std::vector<double4> &img) {
+  int tot = 0;
+  for (int s = 0; s < ns; s++) tot += tables[s].ngrid;
+  // doubles: img | r f fp fpp | a b rmax cut | then ints and floats
+  const size_t nd = 4 * img.size() + 4 * (size_t)tot + 4 * (size_t)ns;
+  const size_t bytes = 8 * nd + 4 * 7 * (size_t)ns;
+  char *h = static_cast<char *>(pinned(ctx, bytes));
+  char *d = buf<char>(ctx, "pm_tables", bytes);
+  double *hd = reinterpret_cast<double *>(h), *dd = reinterpret_cast<double *>(d);
+  int *hi = reinterpret_cast<int *>(h + 8 * nd), *di = reinterpret_cast<int *>(d + 8 * nd);
+  float *hf = reinterpret_cast<float *>(hi + 2 * ns), *df = reinterpret_cast<float *>(di + 2 * ns);
+  const size_t o_r = 4 * img.size(), o_s = o_r + 4 * (size_t)tot;
+  if (!img.empty()) std::memcpy(hd, img.data(), sizeof(double4) * img.size());
+  for (int s = 0, o = 0; s < ns; o += tables[s].ngrid, s++) {
     const c2gpu_radial_table &t = tables[s];
-    std::memcpy(&r[toff[s]], t.r, 8 * t.ngrid);
-    std::memcpy(&f[toff[s]], t.f, 8 * t.ngrid);
-    std::memcpy(&fp[toff[s]], t.fp, 8 * t.ngrid);
-    std::memcpy(&fpp[toff[s]], t.fpp, 8 * t.ngrid);
+    const double *col[4] = {t.r, t.f, t.fp, t.fpp};
+    for (int c = 0; c < 4; c++) std::memcpy(hd + o_r + (size_t)c * tot + o, col[c], 8 * (size_t)t.ngrid);
+    const double cut = t.cutrad < t.rmax ? t.cutrad : t.rmax;
+    hd[o_s + s] = t.a;
+    hd[o_s + ns + s] = t.b;
+    hd[o_s + 2 * ns + s] = t.rmax;
+    hd[o_s + 3 * ns + s] = cut;
+    hi[s] = o;
+    hi[ns + s] = t.ngrid;
+    hf[s] = (float)(1.0 / t.b);
+    hf[ns + s] = (float)std::log(t.a);
+    hf[2 * ns + s] = (float)t.r[0];
+    hf[3 * ns + s] = (float)t.rmax;
+    hf[4 * ns + s] = (float)(cut * cut);
   }
-  // FP32 cubic coefficients per (species, base): expand the Lagrange basis
-  // l_i(r) = prod_{j != i} (r - r_j)/(r_i - r_j) in u = r - r_{base-1}.
-  std::vector<float> coef((size_t)tot * 16, 0.f), node(tot, 0.f);
-  for (int s = 0; s < ns; s++) {
-    const int ng = tng[s];
-    for (int base = 2; base <= ng - 2; base++) {
-      const int o = toff[s];
-      double rr[4];
-      for (int i = 0; i < 4; i++) rr[i] = r[o + base - 2 + i];
-      const double u0 = rr[1];
-      double pc[3][4] = {{0}};
-      for (int i = 0; i < 4; i++) {
-        // polynomial prod_{j != i} (u - (r_j - u0)) / (r_i - r_j)
-        double poly[4] = {1, 0, 0, 0};
-        double den = 1;
-        for (int j = 0; j < 4; j++) {
-          if (j == i) continue;
-          const double root = rr[j] - u0;
-          double np[4] = {0, 0, 0, 0};
-          for (int d = 0; d < 3; d++) {
-            np[d + 1] += poly[d];
-            np[d] -= root * poly[d];
-          }
-          for (int d = 0; d < 4; d++) poly[d] = np[d];
-          den *= (rr[i] - rr[j]);
-        }
-        const int ii = o + base - 2 + i;
-        for (int d = 0; d < 4; d++) {
-          pc[0][d] += f[ii] * poly[d] / den;
-          pc[1][d] += fp[ii] * poly[d] / den;
-          pc[2][d] += fpp[ii] * poly[d] / den;
-        }
-      }
-      for (int tbl = 0; tbl < 3; tbl++)
-        for (int d = 0; d < 4; d++) coef[(size_t)(o + base) * 16 + 4 * tbl + d] = (float)pc[tbl][d];
-      node[o + base] = (float)u0;
-    }
-  }
-  std::vector<float> cut2(ns), tainvb(ns), tloga(ns), tr0(ns), trmaxf(ns);
-  for (int s = 0; s < ns; s++) {
-    cut2[s] = (float)(tcut[s] * tcut[s]);
-    tainvb[s] = (float)(1.0 / tb[s]);
-    tloga[s] = (float)std::log(ta[s]);
-    tr0[s] = (float)r[toff[s]];
-    trmaxf[s] = (float)trmax[s];
-  }
-  auto up = [&](const std::string &name, const void *src, size_t bytes) {
-    void *d = buffer(ctx, name, bytes);
-    C2_HIP(hipMemcpyAsync(d, src, bytes, hipMemcpyHostToDevice, ctx->stream));
-    return d;
-  };
-  P.D.r = (const double *)up("pm_r", r.data(), 8 * tot);
-  P.D.f = (const double *)up("pm_f", f.data(), 8 * tot);
-  P.D.fp = (const double *)up("pm_fp", fp.data(), 8 * tot);
-  P.D.fpp = (const double *)up("pm_fpp", fpp.data(), 8 * tot);
-  P.D.toff = (const int *)up("pm_toff", toff.data(), 4 * ns);
-  P.D.tng = (const int *)up("pm_tng", tng.data(), 4 * ns);
-  P.D.ta = (const double *)up("pm_ta", ta.data(), 8 * ns);
-  P.D.tb = (const double *)up("pm_tb", tb.data(), 8 * ns);
-  P.D.trmax = (const double *)up("pm_trmax", trmax.data(), 8 * ns);
-  P.D.tcut = (const double *)up("pm_tcut", tcut.data(), 8 * ns);
-  P.F.coef = (const float4 *)up("pm_coef", coef.data(), 4 * coef.size());
+  C2_HIP(hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, ctx->stream));
+  double *inv = buf<double>(ctx, "pm_inv", 6 * (size_t)tot);
+  float *coef = buf<float>(ctx, "pm_coef", 16 * (size_t)tot), *node = buf<float>(ctx, "pm_node", tot);
+  PromolDev P;
+  P.img = reinterpret_cast<double4 *>(dd);
+  P.nimg = (int)img.size();
+  P.D.r = dd + o_r;
+  P.D.f = P.D.r + tot;
+  P.D.fp = P.D.f + tot;
+  P.D.fpp = P.D.fp + tot;
+  P.D.ta = dd + o_s;
+  P.D.tb = P.D.ta + ns;
+  P.D.trmax = P.D.tb + ns;
+  P.D.tcut = P.D.trmax + ns;
+  P.D.toff = di;
+  P.D.tng = di + ns;
+  P.D.inv = inv;
+  P.rcut = P.D.tcut;
+  P.F.coef = reinterpret_cast<const float4 *>(coef);
   P.F.toff = P.D.toff;
   P.F.tng = P.D.tng;
-  P.F.ta_inv_b = (const float *)up("pm_tainvb", tainvb.data(), 4 * ns);
-  P.F.tlog_a = (const float *)up("pm_tloga", tloga.data(), 4 * ns);
-  P.F.tr0 = (const float *)up("pm_tr0", tr0.data(), 4 * ns);
-  P.F.trmax = (const float *)up("pm_trmaxf", trmaxf.data(), 4 * ns);
-  P.F.tnode = (const float *)up("pm_node", node.data(), 4 * node.size());
-  P.rcut = (double *)up("pm_rcut", tcut.data(), 8 * ns);
-  P.F.cut2 = (const float *)up("pm_cut2", cut2.data(), 4 * ns);
-  double *inv = buf<double>(ctx, "pm_inv", 6 * (size_t)tot);
-  C2_LAUNCH(ctx, k_table_inv, dim3(grid_for(tot, 256)), dim3(256), 0, tot, P.D.r, inv);
-  P.D.inv = inv;
-  C2_HIP(hipStreamSynchronize(ctx->stream));  // the host vectors end here
-  return rcmax;
+  P.F.ta_inv_b = df;
+  P.F.tlog_a = df + ns;
+  P.F.tr0 = df + 2 * ns;
+  P.F.trmax = df + 3 * ns;
+  P.F.cut2 = df + 4 * ns;
+  P.F.tnode = node;
+  C2_LAUNCH(ctx, k_table_build, dim3(grid_for(tot, 64)), dim3(64), 0, tot, ns, P.D.r, P.D.f, P.D.fp, P.D.fpp,
+            P.D.toff, P.D.tng, inv, coef, node);
+  C2_HIP(hipStreamSynchronize(ctx->stream));  // the staging buffer is free again
+  return P;
 }
 
 // Tables and the atom images of the cell that can reach the nodes (the cell,
@@ -745,20 +772,14 @@ static PromolDev upload_promol(c2gpu_ctx *ctx, const c2gpu_promol *pm, const dou
     fail(C2GPU_ERR_ARG, "c2gpu_nci: promolecular tables required");
   for (int a = 0; a < pm->nat; a++)
     if (pm->species[a] < 0 || pm->species[a] >= pm->nspecies) fail(C2GPU_ERR_ARG, "c2gpu_nci: bad species index");
-  PromolDev P;
-  const double rcmax = upload_tables(ctx, pm->nspecies, pm->tables, P);
+  const double rcmax = table_reach(pm->nspecies, pm->tables);
   std::vector<double> pos;
   std::vector<int> isp, iat;
   expand_images(x2c, pm->nat, pm->xat, pm->species, rcmax, pos, isp, iat, lo, hi);
-  const int nimg = (int)isp.size();
-  std::vector<double4> h_img(nimg > 0 ? nimg : 1);
-  for (int m = 0; m < nimg; m++)
-    h_img[m] = make_double4(pos[3 * m], pos[3 * m + 1], pos[3 * m + 2], (double)isp[m]);
-  P.img = buf<double4>(ctx, "pm_img", h_img.size());
-  C2_HIP(hipMemcpyAsync(P.img, h_img.data(), sizeof(double4) * h_img.size(), hipMemcpyHostToDevice, ctx->stream));
-  C2_HIP(hipStreamSynchronize(ctx->stream));
-  P.nimg = nimg;
-  return P;
+  std::vector<double4> img(isp.size());
+  for (size_t m = 0; m < img.size(); m++)
+    img[m] = make_double4(pos[3 * m], pos[3 * m + 1], pos[3 * m + 2], (double)isp[m]);
+  return upload_tables(ctx, pm->nspecies, pm->tables, img);
 }
 
 #define HIPFFT_CHECK(call)                                                     \
@@ -1258,17 +1279,16 @@ void nci_fragments_run(c2gpu_ctx *ctx, const c2gpu_nci_nodes *nd, int nspecies, 
   }
   const int nat = fstart[nfrag];
   if (nat > 0 && (!xyz || !species)) fail(C2GPU_ERR_ARG, "c2gpu_nci_fragments: NULL atoms");
-  std::vector<double4> h(nat > 0 ? nat : 1);
+  std::vector<double4> h(nat > 0 ? nat : 1, make_double4(0.0, 0.0, 0.0, 0.0));
   for (int a = 0; a < nat; a++) {
     if (species[a] < 0 || species[a] >= nspecies) fail(C2GPU_ERR_ARG, "c2gpu_nci_fragments: bad species index");
     h[a] = make_double4(xyz[3 * a], xyz[3 * a + 1], xyz[3 * a + 2], (double)species[a]);
   }
-  PromolDev P;
-  upload_tables(ctx, nspecies, tables, P);
+  table_reach(nspecies, tables);
+  const PromolDev P = upload_tables(ctx, nspecies, tables, h);
   hipStream_t st = ctx->stream;
-  double4 *d_at = buf<double4>(ctx, "frag_at", h.size());
+  const double4 *d_at = P.img;
   int *d_fs = buf<int>(ctx, "frag_start", fstart.size());
-  C2_HIP(hipMemcpyAsync(d_at, h.data(), sizeof(double4) * h.size(), hipMemcpyHostToDevice, st));
   C2_HIP(hipMemcpyAsync(d_fs, fstart.data(), sizeof(int) * fstart.size(), hipMemcpyHostToDevice, st));
   const uint64_t npts = (uint64_t)G.n1 * G.n2 * G.n3;
   const size_t osz = precision == C2GPU_FP32 ? 4 : 8;
