@@ -1057,7 +1057,7 @@ void nci_run(c2gpu_ctx *ctx, const double *rho, const int n[3], const double x2c
     if (n[c] < 1) fail(C2GPU_ERR_ARG, "c2gpu_nci: bad grid");
   const size_t N = (size_t)n[0] * n[1] * n[2];
   hipStream_t st = ctx->stream;
-  const Geo G = make_geo(n, x2c, scheme == C2GPU_NCI_PROMOL && zfast);
+  const Geo G = make_geo(n, x2c, zfast);
   const size_t osz = out_f32 ? 4 : 8;
   const bool dev = flags & C2GPU_PTR_DEVICE;
   NciOut O;
