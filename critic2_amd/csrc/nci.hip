@@ -62,10 +62,9 @@ __global__ void __launch_bounds__(64) k_brick_list(Geo G, Images I, uint32_t *__
 
 // The images that can reach a brick, in image order, STAGE_CAP at most at a
 // time in LDS: all of the workgroup's 256 threads test an image each, and the
-// hits keep their order (a prefix over the wavefronts' ballots).  Testing every
-// image against every brick here is hidden in the 2.0 ms of the 512^3 FP32
-// kernel (2.0 before, too); lists in memory took two launches of 0.42 ms, a
-// scan and a read-back.
+// hits keep their order (a prefix over the wavefronts' ballots).  The 512^3
+// FP32 kernel takes 2.0 to 2.3 ms with it, 2.0 with lists read from memory;
+// those took two launches of 0.42 ms, a scan and a read-back.
 constexpr int STAGE_CAP = 512;
 struct ImageStage {
   double4 img[STAGE_CAP];
