@@ -75,6 +75,8 @@ void run_chunks(c2gpu_ctx *ctx, size_t bytes, F &&carry) {
     } catch (const Error &e) {
       std::lock_guard<std::mutex> g(mu);
       if (!failed.exchange(true)) first = e;
+    } catch (...) {  // nothing may leave a thread
+      failed.store(true);
     }
   };
   std::vector<std::thread> pool;
@@ -88,6 +90,7 @@ void run_chunks(c2gpu_ctx *ctx, size_t bytes, F &&carry) {
   for (auto &t : pool) t.join();
   if (failed.load()) {
     (void)hipStreamSynchronize(ctx->stream);
+    if (first.code == C2GPU_OK) first = Error{C2GPU_ERR_ALLOC, "host transfer: out of memory"};
     throw first;
   }
 }
