@@ -185,6 +185,7 @@ class Context:
 
     def __init__(self, device: int = 0):
         self.lib = load()
+        self.device = device
         h = C.c_void_p()
         rc = self.lib.c2gpu_ctx_create(C.byref(h), device)
         if rc != OK:
