@@ -24,10 +24,12 @@
 // library plan was made anew on each call (16 ms).  Measured, whole nciplot
 // calls: 256^3 orthorhombic 20.1 -> 0.57 ms (0.61 with the grid's first pass;
 // kernels 143 + 201 + 251 us, 2 TB/s), 135x120x98 triclinic 19.8 -> 0.23 ms,
-// 512^3 6.5 ms.  Against 80-bit transforms the gradient's largest error is
-// that of the 3-D transforms (2e-16 to 4e-16 of the largest gradient; circulant
-// edges 2e-15, before 1e-15), and the error of s in the low-density nodes is
-// 2 to 40 times smaller, since a line's rounding follows that line's values.
+// 512^3 6.5 ms.  Against 80-bit sums the gradient's largest error is that of
+// the 3-D transforms or less: 2e-16 to 4e-16 of the largest gradient, on
+// circulant edges from 11 to 3391 1e-16 to 1.2e-15 (the 3-D transform of the
+// same lines 6e-16 to 4e-15; second derivatives alike), and the error of s in
+// the low-density nodes is 2 to 40 times smaller, since a line's rounding
+// follows that line's values.
 // Lines are transformed in pairs, packed as one complex line (both multipliers
 // commute with the packing).  Edges with factors 2, 3, 5 and 7 take a
 // mixed-radix Stockham transform in LDS, 8 elements a thread; other edges the
@@ -48,6 +50,9 @@ namespace {
 
 constexpr int EPT = 8;          // complex elements a thread owns
 constexpr int MAXT = 512;       // threads of a workgroup
+// Terms of a circulant product summed before they join the total: one chain of
+// n terms loses up to 5e-15 of the result on edges of 3400, sums of 32 1.2e-15.
+constexpr int DENSE_SUM = 32;
 constexpr int MAXEDGE = 3400;   // longest line: n (LW + 2) 16 bytes of LDS at LW = 1
 
 // How the lines of one axis are transformed.
@@ -258,12 +263,17 @@ __device__ __forceinline__ void transform(const AxisPlan &P, const Lane &t, doub
 }
 
 // The axis's constants in LDS: exp(-2 pi i k/n), or the first columns of the
-// circulant matrices of D (x) and S (y).
+// circulant matrices of D (x) and S (y).  Those are taken at the distance
+// q = min(k, n - k) from the diagonal, the sign of the cosine put back: sine
+// and cosine of a rounded k/n near 1 would give the entries next to the
+// diagonal, the largest, a relative error of n 2^-53.
 __device__ __forceinline__ void load_table(const AxisPlan &P, double2 *tw) {
   for (int k = threadIdx.x; k < P.n; k += blockDim.x) {
     double s, c;
     if (P.dense) {
-      sincospi((double)k / (double)P.n, &s, &c);
+      const int q = 2 * k > P.n ? P.n - k : k;
+      sincospi((double)q / (double)P.n, &s, &c);
+      c = q < k ? -c : c;
       const double sg = (k & 1) ? -0.5 : 0.5, n = P.n;
       if (k == 0)
         tw[k] = make_double2(0.0, -(P.n & 1 ? n * n - 1.0 : n * n + 2.0) / 12.0);
@@ -345,18 +355,27 @@ __device__ __forceinline__ void derivatives(const AxisPlan &P, const Lane &t, do
     }
     int nx = i0;  // index of w[0]
     double2 ny = make_double2(0.0, 0.0);
-    for (int j = 0; j < P.n; j++) {
-      const double2 v = z[lds_at<AX>(P, j, t.l)];
+    for (int j0 = 0; j0 < P.n; j0 += DENSE_SUM) {
+      double2 pd[IB] = {}, ps[IB] = {};
+      const int j1 = j0 + DENSE_SUM < P.n ? j0 + DENSE_SUM : P.n;
+      for (int j = j0; j < j1; j++) {
+        const double2 v = z[lds_at<AX>(P, j, t.l)];
+#pragma unroll
+        for (int r = 0; r < IB; r++) {
+          pd[r] = make_double2(pd[r].x + w[r].x * v.x, pd[r].y + w[r].x * v.y);
+          ps[r] = make_double2(ps[r].x + w[r].y * v.x, ps[r].y + w[r].y * v.y);
+        }
+        if (nyq && i0 == 0) ny = (j & 1) ? csub(ny, v) : cadd(ny, v);
+        nx = nx == 0 ? P.n - 1 : nx - 1;
+#pragma unroll
+        for (int r = IB - 1; r > 0; r--) w[r] = w[r - 1];
+        w[0] = tw[nx];
+      }
 #pragma unroll
       for (int r = 0; r < IB; r++) {
-        od[u][r] = make_double2(od[u][r].x + w[r].x * v.x, od[u][r].y + w[r].x * v.y);
-        os[u][r] = make_double2(os[u][r].x + w[r].y * v.x, os[u][r].y + w[r].y * v.y);
+        od[u][r] = cadd(od[u][r], pd[r]);
+        os[u][r] = cadd(os[u][r], ps[r]);
       }
-      if (nyq && i0 == 0) ny = (j & 1) ? csub(ny, v) : cadd(ny, v);
-      nx = nx == 0 ? P.n - 1 : nx - 1;
-#pragma unroll
-      for (int r = IB - 1; r > 0; r--) w[r] = w[r - 1];
-      w[0] = tw[nx];
     }
     if (nyq && i0 == 0) nyq[t.l] = cscale(ny, rn);
   }

@@ -4,8 +4,11 @@ transform beyond it) and over cell shapes, against the oracle's numpy FFT.
 
 The fields are white noise, whose second derivatives are of the size of the
 largest multiplier, so the round-off of either side is a few tens of 2.2e-16
-of the largest value (the circulant sums grow as sqrt(n)): 1e-12 of it is
-asserted."""
+of the largest value: 1e-12 of it is asserted.  The circulant edges are also
+held to the 3-D transform's own round-off, on lines of atom-like peaks and of
+noise, against 80-bit sums."""
+import functools
+
 import numpy as np
 import pytest
 
@@ -65,3 +68,78 @@ def test_cells(ctx, cell, grid):
     cz, sz = gn.nciplot_grid(ctx, f, grid, x2c)
     for z, x in ((cz, crho), (sz, s)):
         assert np.array_equal(z.reshape(grid), x.reshape(grid[::-1]).transpose(2, 1, 0))
+
+
+LD = np.longdouble
+
+
+@functools.lru_cache(None)
+def _circulant(n):
+    """First columns, in 80 bits, of the matrices of d/dx and d2/dx2 on n
+    points of a period 2 pi, summed from their definitions."""
+    k = np.arange(n)
+    pi = 4 * np.arctan(LD(1))
+    sin, cos = np.sin(2 * pi * k / LD(n)), np.cos(2 * pi * k / LD(n))
+    d, s = np.zeros(n, LD), np.zeros(n, LD)
+    for m in range(1, (n + 1) // 2):
+        mk = m * k % n
+        d -= 2 * m * sin[mk]
+        s -= 2 * m * m * cos[mk]
+    if n % 2 == 0:
+        s -= (n // 2) ** 2 * np.where(k % 2, LD(-1), LD(1))
+    return d / n, s / n
+
+
+def _apply(col, f):
+    n = f.size
+    out = np.zeros(n, LD)
+    for j in range(n):
+        out += np.roll(col, j) * f[j]
+    return out
+
+
+def _line(n, kind):
+    rng = np.random.default_rng(n)
+    if kind == "noise":
+        return rng.normal(size=n)
+    f, length = np.zeros(n), 0.19 * n  # bohr
+    for x, z in zip(rng.uniform(size=max(2, n // 30)), rng.choice([1.0, 2.0, 3.0, 4.0], size=max(2, n // 30))):
+        d = np.abs(np.arange(n) / n - x)
+        d = np.minimum(d, 1 - d) * length
+        f += z ** 3 * np.exp(-2 * z * np.sqrt(d * d + 0.01))
+    return f
+
+
+@pytest.mark.parametrize("kind", ["peaks", "noise"])
+@pytest.mark.parametrize("n", [34, 127, 211, 509, 1408, 3391])
+def test_circulant_edges_are_as_exact_as_the_3d_transform(ctx, n, kind):
+    """The same line on each axis of a small grid, and beside an edge of 3500,
+    which takes the 3-D transform.  The circulant sums are of 32 terms at a
+    time, so their error is that of the entries, a few 2.2e-16 of the largest
+    value for any n, and the transform's is 1e-15 to 3e-15: twice the
+    transform's error is allowed, and 1e-15 in any case."""
+    print(f"[case] circulant edge {n} {kind}", flush=True)
+    f = _line(n, kind)
+    col_d, col_s = _circulant(n)
+    b = 2 * np.pi / 8.0
+    want = {_lib.FT_GRAD: np.abs(_apply(col_d, f)) * b, _lib.FT_YY: _apply(col_s, f) * b * b}
+
+    def error(grid, axis, kind):
+        shape = [1, 1, 1]
+        shape[2 - axis] = n  # x fastest
+        full = np.broadcast_to(f.reshape(shape), grid[::-1])
+        x2c = np.diag([8.0 if a == axis else 1e7 for a in range(3)])
+        if kind == _lib.FT_YY:
+            kind = (_lib.FT_XX, _lib.FT_YY, _lib.FT_ZZ)[axis]
+            ref = want[_lib.FT_YY]
+        else:
+            ref = want[kind]
+        got = gb.fft_deriv(ctx, full, grid, x2c, kind).reshape(grid[::-1])
+        return float(np.abs(got - ref.reshape(shape)).max() / np.abs(ref).max())
+
+    for kind_ in (_lib.FT_GRAD, _lib.FT_YY):
+        allowed = max(2 * error((3500, n, 1), 1, kind_), 1e-15)
+        for axis in range(3):
+            grid = [2, 3, 4]
+            grid[axis] = n
+            assert error(tuple(grid), axis, kind_) <= allowed, (kind_, axis)
