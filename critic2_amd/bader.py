@@ -10,6 +10,7 @@ integrated properties.  The arithmetic runs in libc2gpu on the GPU.
 """
 from __future__ import annotations
 
+import math
 from dataclasses import dataclass, field
 
 import numpy as np
@@ -140,12 +141,12 @@ def basin_sums(ctx: Context, labels, nattr: int, fields=()):
 def _check_device_grid(ctx: Context, rho, npts):
     """The library reads npts doubles from a device grid's address: a
     DeviceArray or CUDA tensor that does not hold them is refused here."""
-    if str(rho.dtype).replace("torch.", "") != "float64":
+    if rho.dtype != np.float64 and str(rho.dtype) != "torch.float64":
         raise TypeError(f"a grid in HBM must be float64, not {rho.dtype}")
     if not getattr(rho, "is_contiguous", lambda: True)():
         raise TypeError("a grid in HBM must be contiguous")
-    if int(rho.numel()) < npts:
-        raise ValueError(f"the grid in HBM holds {int(rho.numel())} values, {npts} are needed")
+    if rho.numel() < npts:
+        raise ValueError(f"the grid in HBM holds {rho.numel()} values, {npts} are needed")
     dev = getattr(getattr(rho, "device", None), "index", None)
     if dev is not None and dev != ctx.device:
         raise ValueError(f"the grid is on GPU {dev}, the context on GPU {ctx.device}")
@@ -156,8 +157,9 @@ def fft_deriv(ctx: Context, rho, n, x2c, kind):
     back), or on a grid in HBM (a contiguous float64 DeviceArray or CUDA
     tensor; DeviceArray back)."""
     if hasattr(rho, "data_ptr") and getattr(rho, "is_cuda", True):
-        _check_device_grid(ctx, rho, int(np.prod(n)))
-        out = ctx.empty((int(np.prod(n)),), np.float64)
+        npts = math.prod(int(v) for v in n)
+        _check_device_grid(ctx, rho, npts)
+        out = ctx.empty((npts,), np.float64)
         nn = np.asarray(n, dtype=np.int32)
         x = _lib.mat_f(x2c)
         ctx.check(ctx.lib.c2gpu_fft_deriv(ctx.h, _lib.ptr(rho), nn.ctypes.data, x.ctypes.data, kind,
