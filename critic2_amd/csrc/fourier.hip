@@ -51,8 +51,8 @@ namespace {
 constexpr int EPT = 8;          // complex elements a thread owns
 constexpr int MAXT = 512;       // threads of a workgroup
 // Terms of a circulant product summed before they join the total: one chain of
-// n terms loses up to 5e-15 of the result on edges of 3400, sums of 32 1.2e-15.
-constexpr int DENSE_SUM = 32;
+// n terms loses up to 5e-15 of the result on edges of 3400, sums of 64 1.1e-15.
+constexpr int CIRC_SUM = 64;
 constexpr int MAXEDGE = 3400;   // longest line: n (LW + 2) 16 bytes of LDS at LW = 1
 
 // How the lines of one axis are transformed.
@@ -286,6 +286,77 @@ __device__ __forceinline__ void load_table(const AxisPlan &P, double2 *tw) {
   }
 }
 
+// D and S of the workgroup's lines on a circulant edge: IB neighbouring outputs
+// of a line at a time; the matrices' entries slide through registers as j
+// advances.
+template <int AX>
+__device__ __forceinline__ void circulant(const AxisPlan &P, const Lane &t, double2 *z, const double2 *tw,
+                                          double2 d[EPT], double2 s[EPT], double2 *nyq) {
+  constexpr int IB = 4, NU = EPT / IB, STEP = 8;  // STEP: w is back in place after it
+  double2 od[NU][IB], os[NU][IB];
+#pragma unroll
+  for (int u = 0; u < NU; u++) {
+    const int i0 = (t.j + u * P.tpl) * IB;
+    if (i0 >= P.n) continue;
+    double2 w[IB], pd[IB] = {}, ps[IB] = {};
+#pragma unroll
+    for (int r = 0; r < IB; r++) {
+      od[u][r] = os[u][r] = make_double2(0.0, 0.0);
+      w[r] = tw[(i0 + r) % P.n];
+    }
+    int nx = i0;  // index of w[0]
+    double2 ny = make_double2(0.0, 0.0);
+    auto term = [&](int j) {
+      const double2 v = z[lds_at<AX>(P, j, t.l)];
+#pragma unroll
+      for (int r = 0; r < IB; r++) {
+        pd[r] = make_double2(pd[r].x + w[r].x * v.x, pd[r].y + w[r].x * v.y);
+        ps[r] = make_double2(ps[r].x + w[r].y * v.x, ps[r].y + w[r].y * v.y);
+      }
+      if (nyq && i0 == 0) ny = (j & 1) ? csub(ny, v) : cadd(ny, v);
+      nx = nx == 0 ? P.n - 1 : nx - 1;
+#pragma unroll
+      for (int r = IB - 1; r > 0; r--) w[r] = w[r - 1];
+      w[0] = tw[nx];
+    };
+    auto total = [&]() {
+#pragma unroll
+      for (int r = 0; r < IB; r++) {
+        od[u][r] = cadd(od[u][r], pd[r]);
+        os[u][r] = cadd(os[u][r], ps[r]);
+        pd[r] = ps[r] = make_double2(0.0, 0.0);
+      }
+    };
+    int j = 0;
+    for (; j + STEP <= P.n; j += STEP) {
+#pragma unroll
+      for (int e = 0; e < STEP; e++) term(j + e);
+      if ((j + STEP) % CIRC_SUM == 0) total();
+    }
+    for (; j < P.n; j++) term(j);
+    total();
+    if (nyq && i0 == 0) nyq[t.l] = cscale(ny, 1.0 / (double)P.n);
+  }
+#pragma unroll
+  for (int pass = 0; pass < 2; pass++) {
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < NU; u++) {
+      const int i0 = (t.j + u * P.tpl) * IB;
+#pragma unroll
+      for (int r = 0; r < IB; r++)
+        if (i0 + r < P.n) z[lds_at<AX>(P, i0 + r, t.l)] = pass == 0 ? od[u][r] : os[u][r];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < EPT; q++) {
+      const int k = t.j + q * P.tpl;
+      if (k >= P.n) continue;
+      (pass == 0 ? d : s)[q] = z[lds_at<AX>(P, k, t.l)];
+    }
+  }
+}
+
 // D and S of the workgroup's lines: x[q] are this thread's elements, and so
 // are d[q] and s[q] (s only if wants).  nyq, when not null, receives the
 // lines' P values (the transform at n/2 over n; n even), one packed pair per
@@ -339,64 +410,7 @@ __device__ __forceinline__ void derivatives(const AxisPlan &P, const Lane &t, do
     }
     return;
   }
-  // circulant: IB neighbouring outputs of the line at a time; the matrices'
-  // entries slide through registers as j advances
-  constexpr int IB = 4, NU = EPT / IB;
-  double2 od[NU][IB], os[NU][IB];
-#pragma unroll
-  for (int u = 0; u < NU; u++) {
-    const int i0 = (t.j + u * P.tpl) * IB;
-    if (i0 >= P.n) continue;
-    double2 w[IB];
-#pragma unroll
-    for (int r = 0; r < IB; r++) {
-      od[u][r] = os[u][r] = make_double2(0.0, 0.0);
-      w[r] = tw[(i0 + r) % P.n];
-    }
-    int nx = i0;  // index of w[0]
-    double2 ny = make_double2(0.0, 0.0);
-    for (int j0 = 0; j0 < P.n; j0 += DENSE_SUM) {
-      double2 pd[IB] = {}, ps[IB] = {};
-      const int j1 = j0 + DENSE_SUM < P.n ? j0 + DENSE_SUM : P.n;
-      for (int j = j0; j < j1; j++) {
-        const double2 v = z[lds_at<AX>(P, j, t.l)];
-#pragma unroll
-        for (int r = 0; r < IB; r++) {
-          pd[r] = make_double2(pd[r].x + w[r].x * v.x, pd[r].y + w[r].x * v.y);
-          ps[r] = make_double2(ps[r].x + w[r].y * v.x, ps[r].y + w[r].y * v.y);
-        }
-        if (nyq && i0 == 0) ny = (j & 1) ? csub(ny, v) : cadd(ny, v);
-        nx = nx == 0 ? P.n - 1 : nx - 1;
-#pragma unroll
-        for (int r = IB - 1; r > 0; r--) w[r] = w[r - 1];
-        w[0] = tw[nx];
-      }
-#pragma unroll
-      for (int r = 0; r < IB; r++) {
-        od[u][r] = cadd(od[u][r], pd[r]);
-        os[u][r] = cadd(os[u][r], ps[r]);
-      }
-    }
-    if (nyq && i0 == 0) nyq[t.l] = cscale(ny, rn);
-  }
-#pragma unroll
-  for (int pass = 0; pass < 2; pass++) {
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < NU; u++) {
-      const int i0 = (t.j + u * P.tpl) * IB;
-#pragma unroll
-      for (int r = 0; r < IB; r++)
-        if (i0 + r < P.n) z[lds_at<AX>(P, i0 + r, t.l)] = pass == 0 ? od[u][r] : os[u][r];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < EPT; q++) {
-      const int k = t.j + q * P.tpl;
-      if (k >= P.n) continue;
-      (pass == 0 ? d : s)[q] = z[lds_at<AX>(P, k, t.l)];
-    }
-  }
+  circulant<AX>(P, t, z, tw, d, s, nyq);
 }
 
 // Where the thread's pair of lines lies in the grid: element k at p + k st,

@@ -114,7 +114,7 @@ def _line(n, kind):
 @pytest.mark.parametrize("n", [34, 127, 211, 509, 1408, 3391])
 def test_circulant_edges_are_as_exact_as_the_3d_transform(ctx, n, kind):
     """The same line on each axis of a small grid, and beside an edge of 3500,
-    which takes the 3-D transform.  The circulant sums are of 32 terms at a
+    which takes the 3-D transform.  The circulant sums are of 64 terms at a
     time, so their error is that of the entries, a few 2.2e-16 of the largest
     value for any n, and the transform's is 1e-15 to 3e-15: twice the
     transform's error is allowed, and 1e-15 in any case."""
