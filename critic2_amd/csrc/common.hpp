@@ -53,6 +53,7 @@ struct c2gpu_ctx {
     void *ptr = nullptr;
     hipEvent_t ev = nullptr;
   } stage[STAGE_SLOTS];
+  uint64_t fourier_calls = 0;  // calls of the Fourier line passes, for their note of non-finite grids
   // the surface weights of the last c2gpu_yt call (context buffers
   // yt_ias, yt_woff, yt_wc, yt_wb, yt_ww), for c2gpu_yt_multipoles, as
   // critic2 keeps them in its YT checkpoint for later yt_weights calls

@@ -37,6 +37,7 @@
 // 101: 200 a point and axis, still close to what the pass's bytes cost).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <string>
@@ -86,6 +87,9 @@ struct PassArgs {
   double *a, *bb, *s1, *q[3];
   double *c1, *c2;                      // P_1 f (y,z), P_2 f (x,z)
   const double *e12, *e13, *e23;        // P_1 P_2 f (z), P_1 P_3 f (y), P_2 P_3 f (x), or null
+  // set to `call` by the first pass of a call whose grid holds a NaN or an
+  // infinity, and read by its last
+  unsigned long long *bad, call;
   double *out;                          // WANT_GRAD, WANT_HESS
   NciOut O;                             // WANT_NCI
 };
@@ -457,6 +461,15 @@ __device__ __forceinline__ void load_tile(const AxisPlan &P, const Lane &t, cons
   }
 }
 
+// A NaN or an infinity anywhere in the grid makes every derivative NaN, as it
+// does in the reference's 3-D transform, though a line transform carries it to
+// its own lines only: the first pass, which transforms every line, notes it
+// from each thread's first derivative, NaN or infinite with any of its line.
+__device__ __forceinline__ void note_nonfinite(const PassArgs &A, double2 d) {
+  if (!__builtin_isfinite(d.x) || !__builtin_isfinite(d.y))
+    __hip_atomic_store(A.bad, A.call, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // nci@proc.f90:598-599: crho and s of a node; npos positive diagonal second
 // derivatives (nci@proc.f90:546-564)
 __device__ __forceinline__ void nci_value(double f, double gsq, int npos, double &crho, double &s) {
@@ -525,6 +538,9 @@ __global__ void __launch_bounds__(MAXT) k_line_ortho(PassArgs A) {
 #pragma unroll
   for (int q = 0; q < EPT; q++) d[q] = s[q] = make_double2(0.0, 0.0);
   derivatives<AX>(P, t, z, tw, x, A.want != WANT_GRAD, d, s, nullptr);
+  if (A.first) note_nonfinite(A, d[0]);
+  const bool bad = A.last && !A.first && *A.bad == A.call;
+  const double nan = __builtin_nan("");
 #pragma unroll
   for (int q = 0; q < EPT; q++) {
     const int k = t.j + q * P.tpl;
@@ -533,12 +549,14 @@ __global__ void __launch_bounds__(MAXT) k_line_ortho(PassArgs A) {
     if (A.want == WANT_HESS) {
       double2 h = cscale(s[q], A.ql);
       if (!A.first) h = cadd(h, ld2(A.h, g, o));
+      if (bad) h = make_double2(nan, nan);
       st2(A.last ? A.out : A.h, g, o, h);
       continue;
     }
     const double gx = A.bl * d[q].x, gy = A.bl * d[q].y;
     double2 gs = make_double2(gx * gx, gy * gy);
     if (!A.first) gs = cadd(gs, ld2(A.gsq, g, o));
+    if (bad) gs = make_double2(nan, nan);
     if (A.want == WANT_GRAD) {
       if (A.last)
         st2(A.out, g, o, make_double2(sqrt(gs.x), sqrt(gs.y)));
@@ -557,8 +575,8 @@ __global__ void __launch_bounds__(MAXT) k_line_ortho(PassArgs A) {
       if (g.v1) A.npos[o + g.second] = (int8_t)c1;
     } else {
       const double2 f = ld2(A.f, g, o);  // again: not held through the transforms
-      nci_value(f.x, gs.x, c0, d[q].x, s[q].x);
-      nci_value(f.y, gs.y, c1, d[q].y, s[q].y);
+      nci_value(f.x, gs.x, bad ? 0 : c0, d[q].x, s[q].x);
+      nci_value(f.y, gs.y, bad ? 0 : c1, d[q].y, s[q].y);
     }
   }
   if (A.last && A.want == WANT_NCI) store_nci<AX>(A, tile, group, t, g, z, d, s);
@@ -590,6 +608,9 @@ __global__ void __launch_bounds__(MAXT) k_line_any(PassArgs A) {
   load_tile(P, t, g, A.f, x);
   double *cn = AX == 0 ? A.c1 : AX == 1 ? A.c2 : nullptr;
   derivatives<AX>(P, t, z, tw, x, hess, d, s, cn ? nyq : nullptr);
+  if (AX == 0) note_nonfinite(A, d[0]);
+  const bool bad = AX == 2 && *A.bad == A.call;
+  const double nan = __builtin_nan("");
   if (cn) {  // the packed lines' Nyquist projections, by each pair's first thread
     __syncthreads();
     if (t.j == 0) {
@@ -646,6 +667,7 @@ __global__ void __launch_bounds__(MAXT) k_line_any(PassArgs A) {
           h[w].y = u.y + A.Q[w][2] * s[q].y + 2.0 * (A.Q[w][4] * a.y + A.Q[w][5] * b.y);
         }
     }
+    if (bad) h[0] = h[1] = h[2] = make_double2(nan, nan);
     if (A.want == WANT_HESS) {
       st2(A.out, g, o, h[0]);
       continue;
@@ -658,6 +680,7 @@ __global__ void __launch_bounds__(MAXT) k_line_any(PassArgs A) {
       const double gy = A.b[c] * da.y + A.b[c + 3] * db.y + A.b[c + 6] * d[q].y;
       gs = make_double2(gs.x + gx * gx, gs.y + gy * gy);
     }
+    if (bad) gs = make_double2(nan, nan);
     if (A.want == WANT_GRAD) {
       st2(A.out, g, o, make_double2(sqrt(gs.x), sqrt(gs.y)));
       continue;
@@ -667,6 +690,15 @@ __global__ void __launch_bounds__(MAXT) k_line_any(PassArgs A) {
     nci_value(f.y, gs.y, (h[0].y > 0.0) + (h[1].y > 0.0) + (h[2].y > 0.0), d[q].y, s[q].y);
   }
   if (AX == 2 && A.want == WANT_NCI) store_nci<AX>(A, tile, group, t, g, z, d, s);
+}
+
+// A call of one pass: its derivatives made NaN where the pass noted a NaN or
+// an infinity.
+__global__ void __launch_bounds__(256) k_line_nan(const unsigned long long *bad, unsigned long long call, uint64_t n,
+                                                  double *out) {
+  if (*bad != call) return;
+  for (uint64_t p = (uint64_t)blockIdx.x * 256 + threadIdx.x; p < n; p += (uint64_t)gridDim.x * 256)
+    out[p] = __builtin_nan("");
 }
 
 // out[o] = (1/n) sum_q (-1)^q in[o so + q sq]: one wavefront each
@@ -772,6 +804,11 @@ void fourier_lines_run(c2gpu_ctx *ctx, const double *f, const int n[3], const do
       }
   }
   std::memcpy(A.b, bvec, sizeof A.b);
+  // calls are numbered, so the word is cleared once, not before each call
+  const bool fresh = ctx->bufs.find("fourier_bad") == ctx->bufs.end();
+  A.bad = buf<unsigned long long>(ctx, "fourier_bad", 1);
+  if (fresh) C2_HIP(hipMemsetAsync(A.bad, 0, sizeof *A.bad, ctx->stream));
+  A.call = ++ctx->fourier_calls;
   // Orthorhombic: one Cartesian component per axis, a different one each.
   // Components below 1e-15 of the largest (a right angle's cosine is 6e-17)
   // change the derivatives by less than the transforms' own rounding.
@@ -812,6 +849,9 @@ void fourier_lines_run(c2gpu_ctx *ctx, const double *f, const int n[3], const do
       else
         launch_pass(ctx, "k_line_ortho<2>", k_line_ortho<2>, 2, A);
     }
+    if (m == 1)
+      C2_LAUNCH(ctx, k_line_nan, dim3((unsigned)std::min<size_t>((N + 255) / 256, 2048)), dim3(256), 0,
+                (const unsigned long long *)A.bad, A.call, (uint64_t)N, out);
     return;
   }
   A.a = buf<double>(ctx, "fourier_gsq", N);

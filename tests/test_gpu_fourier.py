@@ -143,3 +143,39 @@ def test_circulant_edges_are_as_exact_as_the_3d_transform(ctx, n, kind):
             grid = [2, 3, 4]
             grid[axis] = n
             assert error(tuple(grid), axis, kind_) <= allowed, (kind_, axis)
+
+
+@pytest.mark.parametrize("value", [np.nan, np.inf, -np.inf])
+@pytest.mark.parametrize("cell", ["ortho", "permuted", "triclinic"])
+@pytest.mark.parametrize("grid", [(12, 14, 18), (11, 9, 26)])
+def test_non_finite_grids(ctx, cell, grid, value):
+    """One NaN or infinity makes every derivative NaN and leaves crho the sign
+    of no positive second derivative, as a 3-D transform does; the next call on
+    a finite grid is as if that one had not been."""
+    print(f"[case] fourier non-finite {cell} {grid} {value}", flush=True)
+    x2c = CELLS[cell]
+    f = 0.1 + np.random.default_rng(1).uniform(size=int(np.prod(grid)))
+    kinds = (_lib.FT_GRAD, _lib.FT_XX, _lib.FT_YY, _lib.FT_ZZ, _lib.FT_LAP)
+    before = [gb.fft_deriv(ctx, f, grid, x2c, k) for k in kinds] + list(gn.nciplot_grid(ctx, f, grid, x2c))
+    for at in (0, f.size // 2 + 3, f.size - 1):
+        bad = f.copy()
+        bad[at] = value
+        for k in kinds:
+            assert np.isnan(gb.fft_deriv(ctx, bad, grid, x2c, k)).all(), (at, k)
+        crho, s = gn.nciplot_grid(ctx, bad, grid, x2c, zfast=False)
+        assert np.isnan(s).all()
+        np.testing.assert_array_equal(crho, -np.abs(bad) * 100.0)
+    after = [gb.fft_deriv(ctx, f, grid, x2c, k) for k in kinds] + list(gn.nciplot_grid(ctx, f, grid, x2c))
+    for a, b in zip(before, after):
+        np.testing.assert_array_equal(a, b)
+
+
+def test_non_finite_grids_of_the_3d_transform(ctx):
+    """The same from the 3-D transform itself."""
+    grid = (3500, 3, 2)
+    f = 0.1 + np.random.default_rng(2).uniform(size=int(np.prod(grid)))
+    f[17] = np.nan
+    assert np.isnan(gb.fft_deriv(ctx, f, grid, TRI, _lib.FT_LAP)).all()
+    crho, s = gn.nciplot_grid(ctx, f, grid, TRI, zfast=False)
+    assert np.isnan(s).all()
+    np.testing.assert_array_equal(crho, -np.abs(f) * 100.0)
