@@ -292,8 +292,8 @@ __device__ __forceinline__ void load_table(const AxisPlan &P, double2 *tw) {
 
 // D and S of the workgroup's lines on a circulant edge: IB neighbouring outputs
 // of a line at a time; the matrices' entries slide through registers as j
-// advances.
-template <int AX>
+// advances.  S: also the second derivatives.
+template <int AX, bool S>
 __device__ __forceinline__ void circulant(const AxisPlan &P, const Lane &t, double2 *z, const double2 *tw,
                                           double2 d[EPT], double2 s[EPT], double2 *nyq) {
   constexpr int IB = 4, NU = EPT / IB, STEP = 8;  // STEP: w is back in place after it
@@ -315,7 +315,7 @@ __device__ __forceinline__ void circulant(const AxisPlan &P, const Lane &t, doub
 #pragma unroll
       for (int r = 0; r < IB; r++) {
         pd[r] = make_double2(pd[r].x + w[r].x * v.x, pd[r].y + w[r].x * v.y);
-        ps[r] = make_double2(ps[r].x + w[r].y * v.x, ps[r].y + w[r].y * v.y);
+        if (S) ps[r] = make_double2(ps[r].x + w[r].y * v.x, ps[r].y + w[r].y * v.y);
       }
       if (nyq && i0 == 0) ny = (j & 1) ? csub(ny, v) : cadd(ny, v);
       nx = nx == 0 ? P.n - 1 : nx - 1;
@@ -342,7 +342,7 @@ __device__ __forceinline__ void circulant(const AxisPlan &P, const Lane &t, doub
     if (nyq && i0 == 0) nyq[t.l] = cscale(ny, 1.0 / (double)P.n);
   }
 #pragma unroll
-  for (int pass = 0; pass < 2; pass++) {
+  for (int pass = 0; pass < (S ? 2 : 1); pass++) {
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < NU; u++) {
@@ -414,7 +414,10 @@ __device__ __forceinline__ void derivatives(const AxisPlan &P, const Lane &t, do
     }
     return;
   }
-  circulant<AX>(P, t, z, tw, d, s, nyq);
+  if (wants)
+    circulant<AX, true>(P, t, z, tw, d, s, nyq);
+  else
+    circulant<AX, false>(P, t, z, tw, d, s, nyq);
 }
 
 // Where the thread's pair of lines lies in the grid: element k at p + k st,
