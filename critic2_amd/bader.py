@@ -301,10 +301,11 @@ def bader(ctx: Context, rho, n, x2c, xat, nnm=False, ratom=None, noatoms=False, 
     grid crosses to the GPU once for the whole keyword, its labels back once."""
     host = not hasattr(rho, "data_ptr")
     if host:
+        npts = math.prod(int(v) for v in n)
         rho = np.ascontiguousarray(rho, dtype=np.float64).reshape(-1)
-        if rho.size != int(np.prod(n)):
-            raise ValueError(f"rho holds {rho.size} values, the grid {tuple(n)} has {int(np.prod(n))}")
-        rho = ctx.to_device(rho)
+        if rho.size < npts:
+            raise ValueError(f"rho holds {rho.size} values, the grid {tuple(n)} has {npts}")
+        rho = ctx.to_device(rho[:npts])
     bas = bader_integrate(ctx, rho, n, x2c, xat, nnm=nnm, ratom=ratom, noatoms=noatoms)
     props = intgrid_fields(ctx, bas, rho, x2c, lap=lap)
     if host:

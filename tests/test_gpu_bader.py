@@ -281,3 +281,17 @@ def test_bader_edge_grids_bit_exact(ctx, name, seed, edge, ang, nat, n, q):
     assert bas.nattr == info["nattr"]
     assert bas.stats["refine_iters"] == info["refine_iters"]
     np.testing.assert_array_equal(bas.xattr, xattr)
+
+
+def test_bader_host_array_longer_than_the_grid(ctx):
+    """A host array is read to the grid's size, whatever follows; a shorter one
+    is refused."""
+    cell = random_cell(11, (9.0, 10.0, 11.0), (78, 97, 105), 6, (1, 6, 7, 8), (20, 22, 24))
+    f = _grid(ctx, cell)
+    bas, props = gb.bader(ctx, f, cell.n, cell.x2c, cell.xat)
+    more, p = gb.bader(ctx, np.concatenate([f, np.full(777, 1e9)]), cell.n, cell.x2c, cell.xat)
+    np.testing.assert_array_equal(more.idg, bas.idg)
+    for k in props:
+        np.testing.assert_array_equal(p[k], props[k])
+    with pytest.raises(ValueError):
+        gb.bader(ctx, f[:-1], cell.n, cell.x2c, cell.xat)
