@@ -8,8 +8,9 @@
 // beside the link.  Measured: a 160 MB cube file read and parsed into HBM
 // 41.6 -> 4.2 ms (two 64 MiB slots made per call before), 386 MB of cube text
 // out of it 110 -> 10.4 ms.  Six threads: a warm destination takes 49 GB/s,
-// and four already read the page cache at 40 GB/s.  The slots (24 MiB) are made on first use, kept by the
-// context and given back with it.
+// and four already read the page cache at 40 GB/s.  The slots (24 MiB) are made
+// on first use, kept by the context and given back with it; where pinned memory
+// runs out the slots there are do the work, and with none the runtime's copy.
 #include <fcntl.h>
 #include <hip/hip_runtime.h>
 #include <sys/stat.h>
@@ -34,30 +35,42 @@ constexpr size_t STAGE_CHUNK = (size_t)4 << 20;  // bytes of a slot
 // below this one runtime copy costs less than starting the threads
 constexpr size_t STAGE_MIN = (size_t)2 << 20;
 
-void stage_slots(c2gpu_ctx *ctx) {
+// The number of slots to be had, the first of the context's: fewer than
+// STAGE_THREADS, or none, where pinned memory runs out.  The missing ones are
+// asked for again by the next transfer.
+int stage_slots(c2gpu_ctx *ctx) {
   for (int i = 0; i < STAGE_THREADS; i++) {
     auto &s = ctx->stage[i];
-    if (!s.ptr) {
-      const hipError_t e = hipHostMalloc(&s.ptr, STAGE_CHUNK, hipHostMallocDefault);
-      if (e != hipSuccess) {
-        s.ptr = nullptr;
-        fail(C2GPU_ERR_ALLOC, std::string("hipHostMalloc(staging): ") + hipGetErrorString(e));
-      }
+    if (!s.ptr && hipHostMalloc(&s.ptr, STAGE_CHUNK, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      s.ptr = nullptr;
+      return i;
     }
     if (!s.ev) C2_HIP(hipEventCreateWithFlags(&s.ev, hipEventDisableTiming));
   }
+  return STAGE_THREADS;
 }
 
+// A slot of ordinary memory, for files where no pinned slot is to be had.
+struct PlainSlot {
+  std::vector<char> mem;
+  c2gpu_ctx::Stage slot;
+  explicit PlainSlot(size_t bytes) : mem(bytes) {
+    slot.ptr = mem.data();
+    C2_HIP(hipEventCreateWithFlags(&slot.ev, hipEventDisableTiming));
+  }
+  ~PlainSlot() { (void)hipEventDestroy(slot.ev); }
+};
+
 // Runs carry(slot, offset, length) for every chunk of [0, bytes), chunks
-// spread over the slots' threads; the first error stops the rest and is
-// rethrown once every thread has ended.
+// spread over a thread for each of the `slots`; the first error stops the rest
+// and is rethrown once every thread has ended.
 template <class F>
-void run_chunks(c2gpu_ctx *ctx, size_t bytes, F &&carry) {
-  stage_slots(ctx);
+void run_chunks(c2gpu_ctx *ctx, c2gpu_ctx::Stage *stage, int slots, size_t bytes, F &&carry) {
   // at least two chunks a thread where the transfer allows it
-  const size_t chunk = std::min(STAGE_CHUNK, std::max((size_t)1 << 19, bytes / (2 * STAGE_THREADS) + 1));
+  const size_t chunk = std::min(STAGE_CHUNK, std::max((size_t)1 << 19, bytes / (2 * slots) + 1));
   const size_t n = (bytes + chunk - 1) / chunk;
-  const int nt = (int)std::min<size_t>(STAGE_THREADS, n);
+  const int nt = (int)std::min<size_t>(slots, n);
   std::atomic<size_t> next{0};
   std::atomic<bool> failed{false};
   std::mutex mu;
@@ -69,9 +82,9 @@ void run_chunks(c2gpu_ctx *ctx, size_t bytes, F &&carry) {
         const size_t c = next.fetch_add(1);
         if (c >= n || failed.load()) break;
         const size_t o = c * chunk;
-        carry(ctx->stage[t], o, std::min(chunk, bytes - o));
+        carry(stage[t], o, std::min(chunk, bytes - o));
       }
-      C2_HIP(hipEventSynchronize(ctx->stage[t].ev));  // the slot is free again
+      C2_HIP(hipEventSynchronize(stage[t].ev));  // the slot is free again
     } catch (const Error &e) {
       std::lock_guard<std::mutex> g(mu);
       if (!failed.exchange(true)) first = e;
@@ -80,7 +93,7 @@ void run_chunks(c2gpu_ctx *ctx, size_t bytes, F &&carry) {
     }
   };
   std::vector<std::thread> pool;
-  pool.reserve(STAGE_THREADS);
+  pool.reserve(slots);
   try {
     for (int t = 1; t < nt; t++) pool.emplace_back(work, t);
   } catch (const std::exception &) {
@@ -92,6 +105,17 @@ void run_chunks(c2gpu_ctx *ctx, size_t bytes, F &&carry) {
     (void)hipStreamSynchronize(ctx->stream);
     if (first.code == C2GPU_OK) first = Error{C2GPU_ERR_ALLOC, "host transfer: out of memory"};
     throw first;
+  }
+}
+
+// run_chunks with the context's slots, or one of ordinary memory.
+template <class F>
+void run_file(c2gpu_ctx *ctx, size_t bytes, F &&carry) {
+  if (const int slots = stage_slots(ctx)) {
+    run_chunks(ctx, ctx->stage, slots, bytes, carry);
+  } else {
+    PlainSlot plain(std::min(STAGE_CHUNK, bytes));
+    run_chunks(ctx, &plain.slot, 1, bytes, carry);
   }
 }
 
@@ -109,11 +133,12 @@ bool pageable(const void *p) {
 
 void copy_in(c2gpu_ctx *ctx, void *dst, const void *src, size_t bytes) {
   if (bytes == 0) return;
-  if (bytes < STAGE_MIN || !pageable(src)) {
+  const int slots = bytes < STAGE_MIN || !pageable(src) ? 0 : stage_slots(ctx);
+  if (slots == 0) {
     C2_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream));
     return;
   }
-  run_chunks(ctx, bytes, [&](c2gpu_ctx::Stage &s, size_t o, size_t n) {
+  run_chunks(ctx, ctx->stage, slots, bytes, [&](c2gpu_ctx::Stage &s, size_t o, size_t n) {
     C2_HIP(hipEventSynchronize(s.ev));
     std::memcpy(s.ptr, static_cast<const char *>(src) + o, n);
     C2_HIP(hipMemcpyAsync(static_cast<char *>(dst) + o, s.ptr, n, hipMemcpyHostToDevice, ctx->stream));
@@ -123,12 +148,13 @@ void copy_in(c2gpu_ctx *ctx, void *dst, const void *src, size_t bytes) {
 
 void copy_out(c2gpu_ctx *ctx, void *dst, const void *src, size_t bytes) {
   if (bytes == 0) return;
-  if (bytes < STAGE_MIN || !pageable(dst)) {
+  const int slots = bytes < STAGE_MIN || !pageable(dst) ? 0 : stage_slots(ctx);
+  if (slots == 0) {
     C2_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
     C2_HIP(hipStreamSynchronize(ctx->stream));
     return;
   }
-  run_chunks(ctx, bytes, [&](c2gpu_ctx::Stage &s, size_t o, size_t n) {
+  run_chunks(ctx, ctx->stage, slots, bytes, [&](c2gpu_ctx::Stage &s, size_t o, size_t n) {
     C2_HIP(hipMemcpyAsync(s.ptr, static_cast<const char *>(src) + o, n, hipMemcpyDeviceToHost, ctx->stream));
     C2_HIP(hipEventRecord(s.ev, ctx->stream));
     C2_HIP(hipEventSynchronize(s.ev));
@@ -137,7 +163,7 @@ void copy_out(c2gpu_ctx *ctx, void *dst, const void *src, size_t bytes) {
 }
 
 void file_in(c2gpu_ctx *ctx, void *dst, int fd, uint64_t from, uint64_t bytes) {
-  run_chunks(ctx, bytes, [&](c2gpu_ctx::Stage &s, size_t o, size_t n) {
+  run_file(ctx, bytes, [&](c2gpu_ctx::Stage &s, size_t o, size_t n) {
     C2_HIP(hipEventSynchronize(s.ev));
     for (size_t got = 0; got < n;) {
       const ssize_t r = pread(fd, static_cast<char *>(s.ptr) + got, n - got, (off_t)(from + o + got));
@@ -151,7 +177,7 @@ void file_in(c2gpu_ctx *ctx, void *dst, int fd, uint64_t from, uint64_t bytes) {
 }
 
 void file_out(c2gpu_ctx *ctx, int fd, uint64_t to, const void *src, uint64_t bytes) {
-  run_chunks(ctx, bytes, [&](c2gpu_ctx::Stage &s, size_t o, size_t n) {
+  run_file(ctx, bytes, [&](c2gpu_ctx::Stage &s, size_t o, size_t n) {
     C2_HIP(hipMemcpyAsync(s.ptr, static_cast<const char *>(src) + o, n, hipMemcpyDeviceToHost, ctx->stream));
     C2_HIP(hipEventRecord(s.ev, ctx->stream));
     C2_HIP(hipEventSynchronize(s.ev));
