@@ -20,7 +20,8 @@
 #include <atomic>
 #include <cerrno>
 #include <cstring>
-#include <mutex>
+#include <exception>
+#include <string>
 #include <thread>
 #include <vector>
 
@@ -73,8 +74,7 @@ void run_chunks(c2gpu_ctx *ctx, c2gpu_ctx::Stage *stage, int slots, size_t bytes
   const int nt = (int)std::min<size_t>(slots, n);
   std::atomic<size_t> next{0};
   std::atomic<bool> failed{false};
-  std::mutex mu;
-  Error first{C2GPU_OK, ""};
+  std::exception_ptr first;  // written by the thread that sets failed
   auto work = [&](int t) {
     try {
       C2_HIP(hipSetDevice(ctx->device));
@@ -85,16 +85,13 @@ void run_chunks(c2gpu_ctx *ctx, c2gpu_ctx::Stage *stage, int slots, size_t bytes
         carry(stage[t], o, std::min(chunk, bytes - o));
       }
       C2_HIP(hipEventSynchronize(stage[t].ev));  // the slot is free again
-    } catch (const Error &e) {
-      std::lock_guard<std::mutex> g(mu);
-      if (!failed.exchange(true)) first = e;
     } catch (...) {  // nothing may leave a thread
-      failed.store(true);
+      if (!failed.exchange(true)) first = std::current_exception();
     }
   };
   std::vector<std::thread> pool;
-  pool.reserve(slots);
   try {
+    pool.reserve(slots);
     for (int t = 1; t < nt; t++) pool.emplace_back(work, t);
   } catch (const std::exception &) {
     // fewer threads than asked for: the others take the chunks
@@ -103,8 +100,13 @@ void run_chunks(c2gpu_ctx *ctx, c2gpu_ctx::Stage *stage, int slots, size_t bytes
   for (auto &t : pool) t.join();
   if (failed.load()) {
     (void)hipStreamSynchronize(ctx->stream);
-    if (first.code == C2GPU_OK) first = Error{C2GPU_ERR_ALLOC, "host transfer: out of memory"};
-    throw first;
+    try {
+      std::rethrow_exception(first);
+    } catch (const Error &) {
+      throw;
+    } catch (const std::exception &e) {  // callers on threads of their own catch Error alone
+      fail(C2GPU_ERR_ALLOC, std::string("host transfer: ") + e.what());
+    }
   }
 }
 

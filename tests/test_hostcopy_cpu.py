@@ -49,7 +49,7 @@ def test_a_full_disk(check):
 
 
 @pytest.mark.parametrize("copies", [0, 4])
-@pytest.mark.parametrize("how", ["hip"])
+@pytest.mark.parametrize("how", ["hip", "throw"])
 def test_a_copy_that_fails(check, how, copies):
     """The first error comes out as the call's status with its message, no
     thread is left, and the context goes on working."""
