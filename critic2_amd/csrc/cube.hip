@@ -730,7 +730,7 @@ void cube_read_run(c2gpu_ctx *ctx, const char *path, int flags, c2gpu_cube_heade
   double *out = out_grid(ctx, flags, f, npts);
   const uint64_t len = fsize - h->data_offset;
   uint8_t *d = buf<uint8_t>(ctx, "cube_text", len + 16);
-  if (len) file_in(ctx, d, fileno(file.fp), h->data_offset, len);
+  if (len) file_in(ctx, d, fileno(file.fp), h->data_offset, len, "short read");
   parse_values(ctx, d, 0, len, h->n, out);
   if (!(flags & C2GPU_PTR_DEVICE))
     copy_out(ctx, f, out, npts * 8);
@@ -756,7 +756,7 @@ void bincube_read_run(c2gpu_ctx *ctx, const char *path, int flags, c2gpu_cube_he
         fail(C2GPU_ERR_FORMAT, "binary cube: end of file");
     } else if (take) {
       const off_t at = ftello(file.fp);
-      file_in(ctx, reinterpret_cast<char *>(f) + got, fileno(file.fp), (uint64_t)at, take);
+      file_in(ctx, reinterpret_cast<char *>(f) + got, fileno(file.fp), (uint64_t)at, take, "binary cube: end of file");
       fseeko(file.fp, at + (off_t)take, SEEK_SET);
     }
     got += take;

@@ -164,13 +164,13 @@ void copy_out(c2gpu_ctx *ctx, void *dst, const void *src, size_t bytes) {
   });
 }
 
-void file_in(c2gpu_ctx *ctx, void *dst, int fd, uint64_t from, uint64_t bytes) {
+void file_in(c2gpu_ctx *ctx, void *dst, int fd, uint64_t from, uint64_t bytes, const char *ends) {
   run_file(ctx, bytes, [&](c2gpu_ctx::Stage &s, size_t o, size_t n) {
     C2_HIP(hipEventSynchronize(s.ev));
     for (size_t got = 0; got < n;) {
       const ssize_t r = pread(fd, static_cast<char *>(s.ptr) + got, n - got, (off_t)(from + o + got));
       if (r < 0 && errno == EINTR) continue;
-      if (r <= 0) fail(C2GPU_ERR_FORMAT, "short read");
+      if (r <= 0) fail(C2GPU_ERR_FORMAT, ends);
       got += (size_t)r;
     }
     C2_HIP(hipMemcpyAsync(static_cast<char *>(dst) + o, s.ptr, n, hipMemcpyHostToDevice, ctx->stream));

@@ -85,7 +85,7 @@ static void file_trip(c2gpu_ctx *ctx, size_t n, unsigned seed) {
   file_out(ctx, fd, 100, dev.data(), n);
   struct stat st;
   REQUIRE(fstat(fd, &st) == 0 && (size_t)st.st_size == 100 + n);
-  file_in(ctx, back.data(), fd, 100, n);
+  file_in(ctx, back.data(), fd, 100, n, "short read");
   (void)hipStreamSynchronize(ctx->stream);
   REQUIRE(back == want);
   close(fd);
@@ -137,14 +137,14 @@ int main(int argc, char **argv) {
       REQUIRE(ftruncate(fd, 30 * MIB - 1) == 0);
       std::string msg;
       try {
-        file_in(&ctx, dev.data(), fd, 0, 30 * MIB);
+        file_in(&ctx, dev.data(), fd, 0, 30 * MIB, "the file ends early");
       } catch (const Error &e) {
         REQUIRE(e.code == C2GPU_ERR_FORMAT);
         msg = e.msg;
       }
-      REQUIRE(!msg.empty());
+      REQUIRE(msg == "the file ends early");
       close(fd);
-      REQUIRE(code_of([&] { file_in(&ctx, dev.data(), -1, 0, 5 * MIB); }) == C2GPU_ERR_FORMAT);
+      REQUIRE(code_of([&] { file_in(&ctx, dev.data(), -1, 0, 5 * MIB, "short read"); }) == C2GPU_ERR_FORMAT);
       all_sizes(&ctx);
     } else if (what == "full") {
       const int fd = open("/dev/full", O_WRONLY);
