@@ -196,9 +196,11 @@ inline void add_kernel_bytes(c2gpu_ctx *ctx, const char *name, double bytes) {
   } while (0)
 
 // Transfers of caller arrays and files, ordered on the context's stream
-// (hostcopy.cpp).  copy_in / file_in return when the source may change,
-// copy_out / file_out when the destination holds the data.  ends: file_in's
-// message where the file has fewer bytes.
+// (hostcopy.cpp).  copy_out / file_out return when the destination holds the
+// data, file_in when the file has been read, copy_in when a pageable source may
+// change: a pinned or registered one is read until the stream has been waited
+// for, as every entry point does before it returns.  ends: file_in's message
+// where the file has fewer bytes.
 void copy_in(c2gpu_ctx *ctx, void *dst, const void *src, size_t bytes);
 void copy_out(c2gpu_ctx *ctx, void *dst, const void *src, size_t bytes);
 void file_in(c2gpu_ctx *ctx, void *dst, int fd, uint64_t from, uint64_t bytes, const char *ends);
