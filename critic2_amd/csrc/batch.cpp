@@ -36,6 +36,7 @@ static void ensure_workers(c2gpu_ctx *ctx, int nw) {
       fail(C2GPU_ERR_HIP, "c2gpu_batch_run: cannot create a worker stream");
     }
     c->own_stream = true;
+    c->stage_of = ctx;
     ctx->subs.push_back(c);
   }
 }

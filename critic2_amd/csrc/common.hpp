@@ -7,6 +7,7 @@
 #include <cstdio>
 #include <cstring>
 #include <map>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -53,6 +54,8 @@ struct c2gpu_ctx {
     void *ptr = nullptr;
     hipEvent_t ev = nullptr;
   } stage[STAGE_SLOTS];
+  std::mutex stage_mu;            // held while they carry a transfer
+  c2gpu_ctx *stage_of = nullptr;  // a batch worker's: the context whose slots it borrows
   uint64_t fourier_calls = 0;  // calls of the Fourier line passes, for their note of non-finite grids
   // the surface weights of the last c2gpu_yt call (context buffers
   // yt_ias, yt_woff, yt_wc, yt_wb, yt_ww), for c2gpu_yt_multipoles, as

@@ -10,6 +10,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <deque>
+#include <map>
 #include <mutex>
 #include <stdexcept>
 
@@ -58,8 +59,14 @@ struct Event {
 inline std::mutex mu;
 inline int pinned_left = -1;  // hipHostMalloc calls that still succeed (-1: all)
 inline int pinned_live = 0;
+inline std::map<const char *, size_t> pinned;
 inline int copies_left = -1;  // hipMemcpyAsync calls that still succeed
 inline bool copies_throw = false;
+inline bool is_pinned(const void *p) {
+  std::lock_guard<std::mutex> g(mu);
+  auto it = pinned.upper_bound(static_cast<const char *>(p));
+  return it != pinned.begin() && (--it, static_cast<const char *>(p) < it->first + it->second);
+}
 inline bool take(int &left) {
   std::lock_guard<std::mutex> g(mu);
   if (left == 0) return false;
@@ -96,11 +103,13 @@ inline hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
   *p = std::malloc(n);
   std::lock_guard<std::mutex> g(stub::mu);
   stub::pinned_live++;
+  stub::pinned[static_cast<char *>(*p)] = n;
   return hipSuccess;
 }
 inline hipError_t hipHostFree(void *p) {
-  std::free(p);
   std::lock_guard<std::mutex> g(stub::mu);
+  stub::pinned.erase(static_cast<char *>(p));
+  std::free(p);
   stub::pinned_live--;
   return hipSuccess;
 }
@@ -113,14 +122,18 @@ inline hipError_t hipStreamSynchronize(hipStream_t s) {
   s->run_to(n);
   return hipSuccess;
 }
-inline hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t st) {
+// A copy from or to pageable host memory has read or written it on return.
+inline hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind kind, hipStream_t st) {
   if (!stub::take(stub::copies_left)) {
     if (stub::copies_throw) throw std::runtime_error("planted");
     return hipErrorInvalidValue;
   }
-  std::lock_guard<std::mutex> g(st->mu);
-  st->todo.push_back({d, s, n});
-  st->enqueued++;
+  {
+    std::lock_guard<std::mutex> g(st->mu);
+    st->todo.push_back({d, s, n});
+    st->enqueued++;
+  }
+  if (!stub::is_pinned(kind == hipMemcpyHostToDevice ? s : d)) return hipStreamSynchronize(st);
   return hipSuccess;
 }
 inline hipError_t hipEventCreate(hipEvent_t *e) {

@@ -62,7 +62,7 @@ static void round_trip(c2gpu_ctx *ctx, size_t n, unsigned seed) {
   const std::vector<char> want = bytes(n, seed);
   std::vector<char> src = want, dev(n), dst(n);
   copy_in(ctx, dev.data(), src.data(), n);
-  if (n >= 2 * MIB && ctx->stage[0].ptr) std::fill(src.begin(), src.end(), 0);  // staged: the source may change now
+  std::fill(src.begin(), src.end(), 0);  // pageable: it may change now
   (void)hipStreamSynchronize(ctx->stream);
   REQUIRE(dev == want);
   copy_out(ctx, dst.data(), dev.data(), n);
@@ -175,6 +175,15 @@ int main(int argc, char **argv) {
       all_sizes(&ctx);
       t.join();
       REQUIRE(stub::pinned_live == 2 * c2gpu_ctx::STAGE_SLOTS);
+    } else if (what == "shared") {  // batch workers: at once, on the slots of one context
+      Ctx a, b, c;
+      a.stage_of = b.stage_of = c.stage_of = &ctx;
+      std::thread ta([&] { all_sizes(&a); }), tb([&] { all_sizes(&b); }), tc([&] { all_sizes(&c); });
+      all_sizes(&ctx);
+      ta.join();
+      tb.join();
+      tc.join();
+      REQUIRE(stub::pinned_live == c2gpu_ctx::STAGE_SLOTS && !a.stage[0].ptr && !b.stage[0].ptr && !c.stage[0].ptr);
     } else {
       return 2;
     }

@@ -58,3 +58,8 @@ def test_a_copy_that_fails(check, how, copies):
 
 def test_two_contexts_at_once(check):
     check("two")
+
+
+def test_batch_workers_share_the_slots(check):
+    """However many workers, one context's slots and threads."""
+    check("shared")
