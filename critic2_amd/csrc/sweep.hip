@@ -376,10 +376,10 @@ __global__ void k_pre_kt(BParams P, uint32_t N, const uint64_t *__restrict__ Win
 
 // Bound by its gathers and atomics: 168 M 64-byte reads and 77 M atomics (all
 // of them at the memory side) a launch at 512^3.  Two neighbouring workgroups
-// (512 points along x) to an XCD and plain loads: 5.50 -> 4.87 ms a launch at
+// (512 points along x) to an XCD and loads at workgroup scope: 5.50 -> 4.87 ms a launch at
 // 512^3, 39 -> 32 us at 64^3.  More neighbours to an XCD cost time (4: 5.8 ms,
-// 32 and more: 7.2 ms, an eighth of the grid: 8.0 ms), and neither the
-// atomics' scope nor loads past the L2 change it.
+// 32 and more: 7.2 ms, an eighth of the grid: 8.0 ms).  The atomics' scope does
+// not change it; loads at agent scope cost 0.2 ms (41 us instead of 33 at 64^3).
 __global__ void k_pre_cover(BParams P, uint32_t N, const uint64_t *__restrict__ toff, const uint32_t *__restrict__ tp,
                             const uint64_t *__restrict__ Wold, uint64_t *__restrict__ W, int cap) {
   const uint32_t s = xcd_block<2>() * blockDim.x + threadIdx.x;
@@ -399,11 +399,12 @@ __global__ void k_pre_cover(BParams P, uint32_t N, const uint64_t *__restrict__ 
     uint64_t w[PRE_CHUNK];
 #pragma unroll
     for (int u = 0; u < PRE_CHUNK; u++) x[u] = q0 + u < len ? traj_at(P, s, tp, o, q0 + u) : 0u;
-    // each path point's Kt and current covering time in one plain load: a
-    // stale (larger) covering time only costs an atomic that changes nothing
+    // each path point's Kt and current covering time in one load, which may be
+    // served by this CU's cache: a stale (larger) covering time only costs an
+    // atomic that changes nothing
 #pragma unroll
     for (int u = 0; u < PRE_CHUNK; u++)
-      w[u] = q0 + u < len ? W[x[u]] : 0ull;
+      w[u] = q0 + u < len ? __hip_atomic_load(&W[x[u]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) : 0ull;
     bool stop = false;
 #pragma unroll
     for (int u = 0; u < PRE_CHUNK; u++) {
