@@ -666,7 +666,11 @@ __global__ void __launch_bounds__(YB) k_yt_w_dense(YtGeo G, const uint32_t *nfp,
               pres[b - 1] = 1;
             }
         }
-        __builtin_amdgcn_wave_barrier();  // the next neighbour reads what this one's lanes wrote
+        // the next neighbour reads what this one's lanes wrote: LDS operations of
+        // a wavefront run in order, and the fences keep the compiler to it
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
       }
       for (int a = s0; a < s1; a++) mine += pres[a];
     }
