@@ -376,10 +376,11 @@ __global__ void k_pre_kt(BParams P, uint32_t N, const uint64_t *__restrict__ Win
 
 // Bound by its gathers and atomics: 168 M 64-byte reads and 77 M atomics (all
 // of them at the memory side) a launch at 512^3.  Two neighbouring workgroups
-// (512 points along x) to an XCD and loads at workgroup scope: 5.50 -> 4.87 ms a launch at
-// 512^3, 39 -> 32 us at 64^3.  More neighbours to an XCD cost time (4: 5.8 ms,
-// 32 and more: 7.2 ms, an eighth of the grid: 8.0 ms).  The atomics' scope does
-// not change it; loads at agent scope cost 0.2 ms (41 us instead of 33 at 64^3).
+// (512 points along x) to an XCD and loads at workgroup scope: 5.50 -> 4.87 ms
+// a launch at 512^3, 39 -> 32 us at 64^3.  More neighbours to an XCD cost time
+// (4: 5.8 ms, 32 and more: 7.2 ms, an eighth of the grid: 8.0 ms).  The
+// atomics' scope does not change it; loads at agent scope cost 0.2 ms (41 us
+// instead of 33 at 64^3).
 __global__ void k_pre_cover(BParams P, uint32_t N, const uint64_t *__restrict__ toff, const uint32_t *__restrict__ tp,
                             const uint64_t *__restrict__ Wold, uint64_t *__restrict__ W, int cap) {
   const uint32_t s = xcd_block<2>() * blockDim.x + threadIdx.x;
