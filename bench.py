@@ -45,11 +45,15 @@ FP32_PEAK_TFLOPS = 157.3
 STEP_BYTES_PER_POINT = 20
 PROMOL_KERNELS = ("k_promol_f", "k_promol_d", "k_promol_f_queue")
 SUMS_KERNELS = ("k_basin_partials", "k_basin_reduce")
-NCI_GRID_KERNELS = ("k_nci_fft_point", "k_spectral", "k_real_to_complex", "k_accum_sq", "k_count_pos",
+# the Fourier scheme's line passes, its 3-D transforms (an edge too long for
+# the lines) and the tricubic scheme
+NCI_GRID_KERNELS = ("k_line_ortho", "k_line_any", "k_line_nan", "k_alternating",
+                    "k_nci_fft_point", "k_spectral", "k_real_to_complex", "k_accum_sq", "k_count_pos",
                     "k_real_part", "k_sqrt", "k_nci_grid")
 
 
 def compulsory_bytes_per_point(name, nfields=1):
+    name = name.split("<")[0]  # of a template's instance
     if name in PROMOL_KERNELS:
         return 8
     if name in SUMS_KERNELS:
@@ -100,6 +104,16 @@ def measured_traffic(kernel):
             if len(t) == 3 and t[0] == "traffic_bytes_per_launch" and t[1] == kernel:
                 return int(t[2])
     return None
+
+
+def copy_probe(ctx):
+    """Runs one streaming kernel of known traffic, the remap of 2^26 int32
+    labels in place (k_relabel), and says what it must read and write."""
+    npts = 1 << 26
+    lab = ctx.to_device(np.ones(npts, dtype=np.int32))
+    to = np.array([2], dtype=np.int32)
+    ctx.check(ctx.lib.c2gpu_relabel(ctx.h, npts, to.ctypes.data, 1, _lib.PTR_DEVICE, lab.data_ptr()), "c2gpu_relabel")
+    return {"copy_probe": "k_relabel", "points": npts, "bytes_read": 4 * npts, "bytes_written": 4 * npts}
 
 
 def species_of(cell):
@@ -552,8 +566,8 @@ def main():
                     help="time the same step with the grid, labels and NCI outputs in host memory "
                          "(PCIe-inclusive rate)")
     ap.add_argument("--copy-probe", action="store_true",
-                    help="run only a streaming kernel of known traffic (k_sqrt of the FFT |grad| grid: "
-                         "8 B read + 8 B written per point, 256^3) to scale rocprof FETCH_SIZE/WRITE_SIZE")
+                    help="run only a streaming kernel of known traffic (k_relabel: 4 B read + 4 B written "
+                         "per label, 2^26 labels) to scale rocprof FETCH_SIZE/WRITE_SIZE")
     args = ap.parse_args()
     if args.gpus != 1:
         print(json.dumps({"error": "this path runs on one GPU; --gpus must be 1"}))
@@ -572,11 +586,7 @@ def main():
         run_host_buffers(ctx, args)
         return
     if args.copy_probe:
-        probe = config(2)
-        f = gb.synth_slater(ctx, probe)
-        gb.fft_deriv(ctx, f, probe.n, probe.x2c, _lib.FT_GRAD)
-        print(json.dumps({"copy_probe": "k_sqrt", "points": probe.npts,
-                          "bytes_read": 8 * probe.npts, "bytes_written": 8 * probe.npts}), flush=True)
+        print(json.dumps(copy_probe(ctx)), flush=True)
         return
     cell = config(args.config, n_override=(args.n,) * 3 if args.config == 3 else None)
     N = cell.npts
