@@ -54,7 +54,10 @@ constexpr int MAXT = 512;       // threads of a workgroup
 // Terms of a circulant product summed before they join the total: one chain of
 // n terms loses up to 5e-15 of the result on edges of 3400, sums of 64 1.1e-15.
 constexpr int CIRC_SUM = 64;
-constexpr int MAXEDGE = 3400;   // longest line: n (LW + 2) 16 bytes of LDS at LW = 1
+// Longest line: a column tile of one pair and the constants, 3 n 16 bytes, fit
+// the LDS.  Mixed radices can need more than MAXT threads before that: edges
+// with a factor 5 above 2560 (n / 5 butterflies) or 3 above 3072 (n / 6).
+constexpr int MAXEDGE = 3400;
 
 // How the lines of one axis are transformed.
 struct AxisPlan {
@@ -775,7 +778,8 @@ void launch_pass(c2gpu_ctx *ctx, const char *name, K kern, int ax, PassArgs &A) 
 
 }  // namespace
 
-// Whether the line passes take a grid with these edges.
+// Whether the line passes take a grid with these edges: none above MAXEDGE, and
+// none whose butterflies need more than MAXT threads.
 bool fourier_lines_ok(const int n[3]) {
   for (int a = 0; a < 3; a++)
     if (n[a] > MAXEDGE || make_axis(n[a]).threads == 0) return false;

@@ -504,7 +504,7 @@ void nci_grid_launch(c2gpu_ctx *ctx, const Geo &G, const double x2c[9], const do
                      const double *d_rho, const NciOut &O);
 
 // line passes of the Fourier scheme (fourier.hip); the 3-D transforms here
-// serve grids with an edge too long for them
+// serve grids with an edge that they do not take
 bool fourier_lines_ok(const int n[3]);
 void fourier_lines_run(c2gpu_ctx *ctx, const double *f, const int n[3], const double bvec[9], int kind, double *out,
                        const NciOut *O);

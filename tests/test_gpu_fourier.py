@@ -31,8 +31,13 @@ GRIDS = [
     (16, 15, 17), (17, 33, 31), (18, 49, 10),      # remainders of the 16-column tiles; primes
     (64, 9, 35), (11, 128, 22), (26, 13, 96),      # circulant edges, even and odd, on each axis
     (512, 6, 5), (3, 640, 4), (6, 5, 1024), (101, 4, 1001),  # fewer line pairs a workgroup
-    (3375, 3, 2), (2, 3, 2048), (3391, 2, 3),      # near the longest line
+    (3375, 3, 2), (2, 3, 2048), (3391, 2, 3),      # 3375 = 5^3 3^3 needs too many threads: the 3-D transform
     (3500, 3, 2),                                  # the 3-D transform
+    # one pair a workgroup: mixed radices with all 512 threads, and circulant
+    # edges up to the longest, whose column tiles fill the LDS
+    (2560, 3, 2), (3, 2560, 2), (3072, 2, 3), (2, 3, 3072), (2, 3391, 3), (3, 2, 3391), (3400, 2, 2), (2, 3400, 3),
+    (3, 2, 3400),
+    (2, 2625, 3), (3087, 2, 3),                    # the first with a factor 5, 3 past 512 threads: the 3-D transform
 ]
 
 
@@ -68,6 +73,13 @@ def test_cells(ctx, cell, grid):
     cz, sz = gn.nciplot_grid(ctx, f, grid, x2c)
     for z, x in ((cz, crho), (sz, s)):
         assert np.array_equal(z.reshape(grid), x.reshape(grid[::-1]).transpose(2, 1, 0))
+
+
+@pytest.mark.parametrize("cell", ["ortho", "triclinic"])
+@pytest.mark.parametrize("grid", [(2560, 2, 3), (2, 3, 3072), (3, 3391, 2), (2, 3, 3400),   # the longest lines
+                                  (3000, 2, 3), (2, 3, 3375), (3500, 3, 2)])                # the 3-D transform
+def test_nci_of_long_edges(ctx, cell, grid):
+    test_cells(ctx, cell, grid)
 
 
 LD = np.longdouble
