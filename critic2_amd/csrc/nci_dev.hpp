@@ -1,4 +1,4 @@
-// Device definitions shared by the NCI sources: the 8x8x4 node bricks, the
+// Device definitions shared by the NCI sources: the bricks of 256 nodes, the
 // output layout of nciplot's crho/cgrad arrays (nci@proc.f90:502-505) and the
 // middle eigenvalue of the Hessian.
 #pragma once
@@ -101,8 +101,11 @@ __device__ inline T eig_mid_t(T h00, T h11, T h22, T h01, T h02, T h12) {
 // Frobenius norm, since d = l (m - l (l1 + l3)).  x = 2e-3 is eight times the
 // closed form's FP32 error, largest (2.3e-4 F) at a double eigenvalue, where
 // acos is flat.  Elsewhere, and for zeros, infinities and NaN, the closed form
-// decides, so the answer is always its own.  About 45 operations instead of an
-// acos and two cosines.
+// decides, so the answer is its own wherever it loses no squares: entries below
+// 1e18 and a traceless part above 1e-18 in FP32, 1e152 and 1e-152 in FP64.  Past
+// that, where no density table in use reaches, the signs settled here are the
+// right ones and the closed form's need not be.  About 45 operations instead of
+// an acos and two cosines.
 template <class T>
 __device__ __forceinline__ bool eig_mid_negative(T h00, T h11, T h22, T h01, T h02, T h12) {
   T mx = fmax(fmax(fmax(fabs(h00), fabs(h11)), fmax(fabs(h22), fabs(h01))), fmax(fabs(h02), fabs(h12)));
