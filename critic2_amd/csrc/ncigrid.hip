@@ -9,7 +9,8 @@
 // where a rounded-below-zero coordinate wraps to 1.0, in the cell at the
 // origin with u = n (the reference evaluates that cell's cubic there).  The
 // node search must therefore round exactly like the reference, and this file
-// is compiled without floating-point contraction.
+// is compiled without floating-point contraction; only contract_stencil, the
+// sums over the stencil of the cell found, turns it on.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
