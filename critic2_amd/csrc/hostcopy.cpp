@@ -153,12 +153,18 @@ bool pageable(const void *p) {
   return a.type == hipMemoryTypeUnregistered;
 }
 
+// Whether a copy is worth staging and its host side allows it.  One with a null
+// pointer is left to the runtime, which turns it into an error.
+bool staged(size_t bytes, const void *dst, const void *src, const void *host) {
+  return bytes >= STAGE_MIN && dst && src && pageable(host);
+}
+
 }  // namespace
 
 void copy_in(c2gpu_ctx *ctx, void *dst, const void *src, size_t bytes) {
   if (bytes == 0) return;
   std::optional<Slots> slots;
-  if (bytes >= STAGE_MIN && pageable(src)) slots.emplace(ctx);
+  if (staged(bytes, dst, src, src)) slots.emplace(ctx);
   if (!slots || !slots->n) {
     C2_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream));
     return;
@@ -174,7 +180,7 @@ void copy_in(c2gpu_ctx *ctx, void *dst, const void *src, size_t bytes) {
 void copy_out(c2gpu_ctx *ctx, void *dst, const void *src, size_t bytes) {
   if (bytes == 0) return;
   std::optional<Slots> slots;
-  if (bytes >= STAGE_MIN && pageable(dst)) slots.emplace(ctx);
+  if (staged(bytes, dst, src, dst)) slots.emplace(ctx);
   if (!slots || !slots->n) {
     C2_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
     C2_HIP(hipStreamSynchronize(ctx->stream));

@@ -124,6 +124,7 @@ inline hipError_t hipStreamSynchronize(hipStream_t s) {
 }
 // A copy from or to pageable host memory has read or written it on return.
 inline hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind kind, hipStream_t st) {
+  if (!d || !s) return hipErrorInvalidValue;
   if (!stub::take(stub::copies_left)) {
     if (stub::copies_throw) throw std::runtime_error("planted");
     return hipErrorInvalidValue;

@@ -146,6 +146,15 @@ int main(int argc, char **argv) {
       close(fd);
       REQUIRE(code_of([&] { file_in(&ctx, dev.data(), -1, 0, 5 * MIB, "short read"); }) == C2GPU_ERR_FORMAT);
       all_sizes(&ctx);
+    } else if (what == "null") {
+      std::vector<char> a(30 * MIB);
+      for (size_t n : {(size_t)1000, a.size()}) {
+        REQUIRE(code_of([&] { copy_in(&ctx, a.data(), nullptr, n); }) == C2GPU_ERR_HIP);
+        REQUIRE(code_of([&] { copy_in(&ctx, nullptr, a.data(), n); }) == C2GPU_ERR_HIP);
+        REQUIRE(code_of([&] { copy_out(&ctx, a.data(), nullptr, n); }) == C2GPU_ERR_HIP);
+        REQUIRE(code_of([&] { copy_out(&ctx, nullptr, a.data(), n); }) == C2GPU_ERR_HIP);
+      }
+      all_sizes(&ctx);
     } else if (what == "full") {
       const int fd = open("/dev/full", O_WRONLY);
       REQUIRE(fd >= 0);

@@ -44,6 +44,11 @@ def test_a_file_that_ends_early(check):
     check("short")
 
 
+def test_null_pointers(check):
+    """An error of the runtime, whatever the size; nothing is read or written."""
+    check("null")
+
+
 def test_a_full_disk(check):
     check("full")
 
