@@ -812,9 +812,8 @@ void fourier_lines_run(c2gpu_ctx *ctx, const double *f, const int n[3], const do
   }
   std::memcpy(A.b, bvec, sizeof A.b);
   // calls are numbered, so the word is cleared once, not before each call
-  const bool fresh = ctx->bufs.find("fourier_bad") == ctx->bufs.end();
   A.bad = buf<unsigned long long>(ctx, "fourier_bad", 1);
-  if (fresh) C2_HIP(hipMemsetAsync(A.bad, 0, sizeof *A.bad, ctx->stream));
+  if (ctx->fourier_calls == 0) C2_HIP(hipMemsetAsync(A.bad, 0, sizeof *A.bad, ctx->stream));
   A.call = ++ctx->fourier_calls;
   // Orthorhombic: one Cartesian component per axis, a different one each.
   // Components below 1e-15 of the largest (a right angle's cosine is 6e-17)
