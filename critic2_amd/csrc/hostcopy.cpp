@@ -35,8 +35,11 @@ namespace {
 
 constexpr int STAGE_THREADS = c2gpu_ctx::STAGE_SLOTS;
 constexpr size_t STAGE_CHUNK = (size_t)4 << 20;  // bytes of a slot
-// below this one runtime copy costs less than starting the threads
-constexpr size_t STAGE_MIN = (size_t)2 << 20;
+// Below these the runtime's copy is the faster: starting the threads takes 0.1
+// ms.  From and to memory that no cache holds, runtime against staged, in us: in
+// 2 MiB 109, 170; 8 MiB 320, 430; 16 MiB 603, 615; 24 MiB 885, 790; out 2 MiB
+// 123, 175; 4 MiB 248, 285; 6 MiB 372, 385; 8 MiB 486, 426.
+constexpr size_t STAGE_MIN_IN = (size_t)16 << 20, STAGE_MIN_OUT = (size_t)7 << 20;
 
 // The number of slots to be had, the first of the context's: fewer than
 // STAGE_THREADS, or none, where pinned memory runs out.  The missing ones are
@@ -155,8 +158,8 @@ bool pageable(const void *p) {
 
 // Whether a copy is worth staging and its host side allows it.  One with a null
 // pointer is left to the runtime, which turns it into an error.
-bool staged(size_t bytes, const void *dst, const void *src, const void *host) {
-  return bytes >= STAGE_MIN && dst && src && pageable(host);
+bool staged(size_t bytes, size_t least, const void *dst, const void *src, const void *host) {
+  return bytes >= least && dst && src && pageable(host);
 }
 
 }  // namespace
@@ -164,7 +167,7 @@ bool staged(size_t bytes, const void *dst, const void *src, const void *host) {
 void copy_in(c2gpu_ctx *ctx, void *dst, const void *src, size_t bytes) {
   if (bytes == 0) return;
   std::optional<Slots> slots;
-  if (staged(bytes, dst, src, src)) slots.emplace(ctx);
+  if (staged(bytes, STAGE_MIN_IN, dst, src, src)) slots.emplace(ctx);
   if (!slots || !slots->n) {
     C2_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream));
     return;
@@ -180,7 +183,7 @@ void copy_in(c2gpu_ctx *ctx, void *dst, const void *src, size_t bytes) {
 void copy_out(c2gpu_ctx *ctx, void *dst, const void *src, size_t bytes) {
   if (bytes == 0) return;
   std::optional<Slots> slots;
-  if (staged(bytes, dst, src, dst)) slots.emplace(ctx);
+  if (staged(bytes, STAGE_MIN_OUT, dst, src, dst)) slots.emplace(ctx);
   if (!slots || !slots->n) {
     C2_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
     C2_HIP(hipStreamSynchronize(ctx->stream));

@@ -56,7 +56,7 @@ static std::vector<char> bytes(size_t n, unsigned seed) {
 }
 
 constexpr size_t MIB = (size_t)1 << 20;
-static const size_t SIZES[] = {1, 2 * MIB - 1, 2 * MIB, 2 * MIB + 1, 6 * MIB + 3, 24 * MIB + 1, 30 * MIB - 7};
+static const size_t SIZES[] = {1, 2 * MIB, 7 * MIB - 1, 7 * MIB, 7 * MIB + 3, 16 * MIB - 1, 16 * MIB, 26 * MIB - 7};
 
 static void round_trip(c2gpu_ctx *ctx, size_t n, unsigned seed) {
   const std::vector<char> want = bytes(n, seed);
@@ -147,7 +147,7 @@ int main(int argc, char **argv) {
       REQUIRE(code_of([&] { file_in(&ctx, dev.data(), -1, 0, 5 * MIB, "short read"); }) == C2GPU_ERR_FORMAT);
       all_sizes(&ctx);
     } else if (what == "null") {
-      std::vector<char> a(30 * MIB);
+      std::vector<char> a(40 * MIB);
       for (size_t n : {(size_t)1000, a.size()}) {
         REQUIRE(code_of([&] { copy_in(&ctx, a.data(), nullptr, n); }) == C2GPU_ERR_HIP);
         REQUIRE(code_of([&] { copy_in(&ctx, nullptr, a.data(), n); }) == C2GPU_ERR_HIP);

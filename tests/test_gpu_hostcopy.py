@@ -23,6 +23,11 @@ def test_round_trip(ctx, nbytes):
     d.free()
 
 
+@pytest.mark.parametrize("nbytes", [7 * MIB - 1, 7 * MIB, 16 * MIB - 1, 16 * MIB, 16 * MIB + 1])
+def test_round_trip_where_staging_begins(ctx, nbytes):
+    test_round_trip(ctx, nbytes)
+
+
 def test_cube_to_a_pipe(ctx, tmp_path):
     """A destination that cannot be written out of order gets the same bytes."""
     n = (40, 50, 60)
